@@ -16,7 +16,7 @@ HERE = os.path.dirname(os.path.abspath(__file__))
 CSRC = os.path.join(HERE, "csrc")
 BUILD = os.path.join(HERE, "_build")
 LIB = os.path.join(HERE, "libllmario_hip.so")
-SOURCES = ["host.cpp", "plan.cpp", "sched.cpp", "sha256.cpp", "kv_kernels.hip", "decode.hip", "prefill.hip"]
+SOURCES = ["host.cpp", "plan.cpp", "sched.cpp", "sha256.cpp", "kv_kernels.hip", "decode.hip", "prefill.hip", "units.hip"]
 # host-only sources (no device code): compiled as plain C++ by the same compiler
 HOST_ONLY = {"plan.cpp", "sched.cpp", "sha256.cpp"}
 ARCH = os.environ.get("LMH_OFFLOAD_ARCH", "gfx950")

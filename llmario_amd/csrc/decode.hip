@@ -57,8 +57,8 @@ constexpr int waves_per_eu() {
 // steps, not k dependent ones); every lane then folds the item's nh * k partial rows, up to
 // PF_MERGE_ROWS loads in flight (the planner keeps nh * k within that, or nh = 1; nh * K
 // <= 64 follows), into its NP dims, storing a head after its last piece, RB rows at a time (16
-// when no item has more: the lighter kernel runs more waves per SIMD). Prompt merges exist only
-// for hdv = 64 or 128 (the prefill's widths), i.e. hdv = 64 * NP.
+// when no item has more: the lighter kernel runs more waves per SIMD). hdv is a multiple of 4 up to
+// 64 * NP; lanes past it re-read the row's first dims and store nothing.
 template <int NP, int RB>
 __device__ void merge_heads(const RowGeom& r, uint32_t hdv, const MergeItem& mi, const float* part, float* out,
                             uint32_t lane) {
@@ -83,17 +83,19 @@ __device__ void merge_heads(const RowGeom& r, uint32_t hdv, const MergeItem& mi,
     float acc[NP];
 #pragma unroll
     for (int i = 0; i < NP; i++) acc[i] = 0.f;
-    // (head, piece) of row j0 + t, advanced row by row (scalar: no division in the loops). hdv is
-    // 64 * NP here, so every lane loads its NP dims of a row as one vector; rows past the item's
-    // last re-read that row (in bounds, no branch between the loads) and are not folded.
+    // (head, piece) of row j0 + t, advanced row by row (scalar: no division in the loops). Every lane
+    // loads its NP dims of a row as one vector; rows past the item's last re-read that row (in
+    // bounds, no branch between the loads) and are not folded.
     typedef float fv __attribute__((ext_vector_type(NP)));
+    const bool lane_on = lane * NP < hdv;
+    const uint32_t d0 = lane_on ? lane * NP : 0;
     uint32_t h_at = 0, s_at = 0;
     for (uint32_t j0 = 0; j0 < nrow; j0 += RB) {
       fv pre[RB];
       uint32_t h = h_at, sp = s_at;
 #pragma unroll
       for (int t = 0; t < RB; t++) {
-        pre[t] = *(const fv*)(base + (size_t)sp * stride + (size_t)h * hstride + lane * NP);
+        pre[t] = *(const fv*)(base + (size_t)sp * stride + (size_t)h * hstride + d0);
         if (j0 + t + 1 < nrow && ++sp == k) {
           sp = 0;
           h++;
@@ -114,7 +116,9 @@ __device__ void merge_heads(const RowGeom& r, uint32_t hdv, const MergeItem& mi,
               o[i] = acc[i] * iv;
               acc[i] = 0.f;
             }
-            *(fv*)(out + ((size_t)mi.row * r.n_head + mi.kvh * r.group + mi.h0 + h_at) * hdv + lane * NP) = o;
+            // a caller's array: any float address
+            typedef float fvu __attribute__((ext_vector_type(NP), aligned(4)));
+            if (lane_on) *(fvu*)(out + ((size_t)mi.row * r.n_head + mi.kvh * r.group + mi.h0 + h_at) * hdv + d0) = o;
             s_at = 0;
             h_at++;
           }
@@ -858,7 +862,7 @@ hipError_t launch_merge(const RowGeom& r, uint32_t hdv, const MergeItem* items, 
                         uint32_t max_pf_rows, const float* part, float* out, uint32_t max_split, hipStream_t s,
                         const LaunchEv& ev) {
   if (n_items == 0) return hipSuccess;
-  if (hdv == 0 || hdv > ROWS_MAX_DIM || n_pf > n_items || (n_pf > 0 && hdv != 64 && hdv != 128))
+  if (hdv == 0 || hdv > ROWS_MAX_DIM || n_pf > n_items || (n_pf > 0 && (hdv > 256 || hdv % 4)))
     return hipErrorInvalidValue;
   // the prompt tokens' merges and the decode merges as two launches when the call has both (the
   // timing events then bracket the pair)
@@ -868,10 +872,13 @@ hipError_t launch_merge(const RowGeom& r, uint32_t hdv, const MergeItem* items, 
     const dim3 grid((n_pf + 3) / 4), block(256);
     if (max_pf_rows > 64) return hipErrorInvalidValue;   // nh * k <= PF_MERGE_ROWS, or nh = 1 and k <= 64
     const bool light = max_pf_rows <= 16;
-    if (hdv == 64 && light) LMH_LAUNCH(ev_pf, (merge_prompt_kernel<1, 16>), grid, block, 0, s, r, hdv, items, n_pf, part, out);
-    else if (hdv == 64) LMH_LAUNCH(ev_pf, (merge_prompt_kernel<1, PF_MERGE_ROWS>), grid, block, 0, s, r, hdv, items, n_pf, part, out);
-    else if (light) LMH_LAUNCH(ev_pf, (merge_prompt_kernel<2, 16>), grid, block, 0, s, r, hdv, items, n_pf, part, out);
-    else LMH_LAUNCH(ev_pf, (merge_prompt_kernel<2, PF_MERGE_ROWS>), grid, block, 0, s, r, hdv, items, n_pf, part, out);
+#define LMH_PF_MERGE(NP)                                                                                          \
+  if (light) LMH_LAUNCH(ev_pf, (merge_prompt_kernel<NP, 16>), grid, block, 0, s, r, hdv, items, n_pf, part, out); \
+  else LMH_LAUNCH(ev_pf, (merge_prompt_kernel<NP, PF_MERGE_ROWS>), grid, block, 0, s, r, hdv, items, n_pf, part, out)
+    if (hdv <= 64) { LMH_PF_MERGE(1); }
+    else if (hdv <= 128) { LMH_PF_MERGE(2); }
+    else { LMH_PF_MERGE(4); }
+#undef LMH_PF_MERGE
     const hipError_t e = hipGetLastError();
     if (e != hipSuccess || n_dec == 0) return e;
   }

@@ -89,6 +89,16 @@ struct PrefillGeom {
   uint32_t* q_flag;  // workgroup 0 records whether its first unit's Q has bits below the page type
 };
 
+// A unit launch (units.hip).
+struct UnitGeom {
+  uint32_t n_head, group;
+  float scale_log2;  // scale * log2(e)
+  uint32_t window;   // 0 = none
+  uint32_t ng;       // heads per partial slot (units that are key pieces write partials)
+  uint32_t shared;   // 1: some unit of the launch is shared between waves (LDS for their partials)
+  float* part;       // the call's partial slots
+};
+
 // Fused per-row tail of attention_block (see lmh_qk_rope_store): flags as LMH_ROPE_*.
 struct RopeGeom {
   uint32_t n_head, q_stride, flags, half_rot;  // half_rot: rotated pairs (0 = no rotation)
@@ -188,6 +198,13 @@ hipError_t launch_mixed(const PageGeom& g, const PrefillGeom& pg, const PrefillI
                         uint32_t per_wg, uint32_t max_pages, const RowGeom& r, const DecodeItem* items,
                         uint32_t n_items, const float* q, float* out, float* part, const MergeCopy& mc,
                         hipStream_t s, const LaunchEv& ev = {});
+// Units (units.hip) of up to 16 * nb columns (nb 1 or 2): n_wg workgroups of w waves, a UnitWave each.
+// unit_waves: the most waves of a workgroup, 0 where no instance takes the geometry (blocks of 16
+// positions or more). unit_waves_per_cu: what a CU's registers hold at once (occupancy query).
+uint32_t unit_waves(uint32_t kv_type, uint32_t hd, uint32_t hdv, uint32_t layout, uint32_t nb);
+uint32_t unit_waves_per_cu(uint32_t kv_type, uint32_t hd, uint32_t hdv, uint32_t layout, uint32_t nb);
+hipError_t launch_units(const PageGeom& g, const UnitGeom& u, uint32_t nb, uint32_t w, const UnitWave* waves, uint32_t n_wg,
+                        const float* q, float* out, const MergeCopy& mc, hipStream_t s, const LaunchEv& ev = {});
 uint32_t prefill_wg_per_cu();     // prefill workgroups a CU holds when their LDS fits (160 KiB / this)
 uint32_t prefill_cols_per_unit();
 // LDS the prefill kernels declare statically, beside prefill_lds_bytes() of dynamic LDS

@@ -258,6 +258,7 @@ struct lmh_kv {
   int device = 0;
   uint32_t n_cu = 0;                        // compute units of the device
   std::vector<uint32_t> decode_capacity;    // per layer: decode items resident at once (0 = not yet asked)
+  std::vector<std::array<uint32_t, 2>> unit_res;   // per layer: unit waves a CU holds (0 = not yet asked)
   uint8_t* d_pool = nullptr;
   int32_t* d_table = nullptr;
   std::vector<int32_t> h_table;
@@ -863,6 +864,7 @@ int32_t lmh_kv_create(const lmh_kv_options* o, lmh_kv** out) {
   if (e == hipSuccess) e = hipDeviceGetAttribute(&n_cu, hipDeviceAttributeMultiprocessorCount, o->device);
   kv->n_cu = (uint32_t)std::max(n_cu, 1);
   kv->decode_capacity.assign(kv->layers.size(), 0);
+  kv->unit_res.assign(kv->layers.size(), {0, 0});
   if (e == hipSuccess) e = hipMalloc((void**)&kv->d_pool, kv->pool_blocks * kv->block_bytes);
   if (e == hipSuccess) e = hipMalloc((void**)&kv->d_table, std::max<uint64_t>(kv->h_table.size(), 1) * 4);
   if (e == hipSuccess && kv->window) e = hipMalloc((void**)&kv->d_wpool, kv->wpool_blocks * kv->wblock_bytes);
@@ -1386,7 +1388,8 @@ int32_t lmh_qk_rope_store(lmh_kv* kv, uint32_t layer, const lmh_seg* segs, uint6
 }
 
 // What the planner needs to know of the kernel modules for a layer's geometry.
-static void fill_kernel_facts(PlanIn& in, uint32_t kv_type, uint32_t hd, uint32_t hdv, uint32_t group) {
+static void fill_kernel_facts(PlanIn& in, uint32_t kv_type, uint32_t hd, uint32_t hdv, uint32_t group, uint32_t layout) {
+  for (uint32_t nb = 1; nb <= 2; nb++) in.unit_w[nb - 1] = unit_waves(kv_type, hd, hdv, layout, nb);
   in.prefill_supported = prefill_supported(kv_type, hd, hdv, group);
   in.unit_cols = prefill_cols_per_unit();
   in.prefill_wg_per_cu = prefill_wg_per_cu();
@@ -1456,7 +1459,13 @@ static int32_t attend_impl(lmh_kv* kv, uint32_t layer, const lmh_seg* segs, uint
   pin.prefill_no_split = kv->prefill_whole_units;
   pin.noalloc = noalloc;
   pin.noalloc_bytes = NOALLOC_SCRATCH_BYTES;
-  fill_kernel_facts(pin, kv->kv_type, y.hd, y.hdv, group);
+  fill_kernel_facts(pin, kv->kv_type, y.hd, y.hdv, group, y.layout);
+  for (uint32_t nb = 1; nb <= 2; nb++) {
+    if (!pin.unit_w[nb - 1]) continue;
+    uint32_t& n = kv->unit_res[layer][nb - 1];
+    if (n == 0) n = unit_waves_per_cu(kv->kv_type, y.hd, y.hdv, y.layout, nb);
+    pin.unit_waves_per_cu[nb - 1] = n;
+  }
   PlanOut& pl = kv->plan;
   plan_attend(pin, pl);
   const uint32_t ng = pl.ng, slots = pl.slots, pf_wg = pl.pf_wg, pf_per_wg = pl.pf_per_wg, max_pages = pl.max_pages;
@@ -1467,7 +1476,9 @@ static int32_t attend_impl(lmh_kv* kv, uint32_t layer, const lmh_seg* segs, uint
   const size_t items_pad = (items_bytes + 255) / 256 * 256;
   const size_t merges_bytes = kv->plan.merges.size() * sizeof(MergeItem);
   const size_t merges_pad = (merges_bytes + 255) / 256 * 256;
-  // one staged payload: [decode items | merges | prefill items]
+  // one staged payload: [decode items | merges | prefill items], or [merges | unit waves], the latter
+  // copied to the staging slot straight from the plan
+  const size_t uwaves_bytes = kv->plan.uwaves.size() * sizeof(UnitWave);
   kv->payload.resize(items_pad + merges_pad + kv->plan.pitems.size() * sizeof(PrefillItem));
   if (items_bytes) std::memcpy(kv->payload.data(), kv->plan.items.data(), items_bytes);
   if (merges_bytes) std::memcpy(kv->payload.data() + items_pad, kv->plan.merges.data(), merges_bytes);
@@ -1497,7 +1508,8 @@ static int32_t attend_impl(lmh_kv* kv, uint32_t layer, const lmh_seg* segs, uint
       merge_dst = (uint32_t*)kv->merge_buf.p;
     }
   }
-  if ((rc = kv->stage_rows(kv->payload.data(), kv->payload.size(), nullptr, 0, rs, rp, ex, slot, !noalloc)) != LMH_OK)
+  if ((rc = kv->stage_rows(kv->payload.data(), kv->payload.size(), kv->plan.uwaves.data(), uwaves_bytes, rs, rp, ex, slot,
+                           !noalloc)) != LMH_OK)
     return rc;
   const PageGeom g = kv->geom(layer);
   RowGeom r{};
@@ -1550,6 +1562,13 @@ static int32_t attend_impl(lmh_kv* kv, uint32_t layer, const lmh_seg* segs, uint
                       ev);
     if (e != hipSuccess) return kv->hip_fail(e, "decode kernel");
   }
+  if (uwaves_bytes) {
+    const UnitGeom ug{y.n_head, group, r.scale_log2, r.window, ng, pl.u_shared ? 1u : 0u, part};
+    if ((e = time_launch(LMH_KERNEL_PREFILL, ev)) != hipSuccess) return kv->hip_fail(e, "event");
+    e = launch_units(g, ug, pl.u_nb, pl.u_w, (const UnitWave*)(ex + items_pad + merges_pad), (uint32_t)(pl.uwaves.size() / pl.u_w),
+                     q, out, mc, st, ev);
+    if (e != hipSuccess) return kv->hip_fail(e, "unit kernel");
+  }
   if (!kv->plan.merges.empty()) {
     if ((e = time_launch(LMH_KERNEL_MERGE, ev)) != hipSuccess) return kv->hip_fail(e, "event");
     // the planner lists the prompt tokens' merges (nh != 0) before the decode merges
@@ -1558,7 +1577,7 @@ static int32_t attend_impl(lmh_kv* kv, uint32_t layer, const lmh_seg* segs, uint
       if (m.nh != 0) {
         max_pf_rows = std::max(max_pf_rows, m.nh * m.n_split);
         if (n_pf != (uint32_t)(&m - kv->plan.merges.data()) || m.n_split > PF_MAX_PIECES ||
-            (m.nh > 1 && m.nh * m.n_split > PF_MERGE_ROWS) || (y.hdv != 64 && y.hdv != 128))
+            (m.nh > 1 && m.nh * m.n_split > PF_MERGE_ROWS) || y.hdv > 256 || y.hdv % 4)
           return kv->fail(LMH_UNSUPPORTED, "attend: the planner's prompt merges are out of order or too long");
         n_pf++;
       } else {
@@ -1676,7 +1695,8 @@ int32_t lmh_plan_attend(const lmh_plan_desc* d, const lmh_seg* segs, uint64_t n_
   in.prefill_no_split = d->tuning.prefill_whole_units != 0;
   in.noalloc = d->noalloc != 0;
   in.noalloc_bytes = NOALLOC_SCRATCH_BYTES;
-  fill_kernel_facts(in, d->kv_type, d->hd, d->hdv, d->n_head / d->n_kv);
+  in.list_units = true;
+  fill_kernel_facts(in, d->kv_type, d->hd, d->hdv, d->n_head / d->n_kv, in.layout);
   PlanOut o;
   if (n_rows > 0) plan_attend(in, o);
   counts->n_items = o.items.size();

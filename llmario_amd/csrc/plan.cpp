@@ -74,6 +74,298 @@ struct WgLists {
   }
 };
 
+// A cut unit's merges: per token over the unit's heads of that token, in groups of heads whose
+// partial rows (heads x k pieces) one merge wave loads at once: f(token, first head, heads) for each.
+// At most `heads` at a time.
+template <typename F>
+void for_each_merge(const PrefillItem& it, uint64_t group, uint32_t k, F&& f, uint32_t heads = PF_MERGE_ROWS) {
+  const uint32_t hpm = std::max<uint32_t>(1, std::min(heads, PF_MERGE_ROWS / k));
+  const uint64_t c_abs = it.c_off;   // the unit's first column, counted from its first token
+  for (uint32_t i = 0; i < it.n_tok; i++) {
+    const uint64_t h_lo = i == 0 ? c_abs : 0;
+    const uint64_t h_hi = std::min<uint64_t>(group, c_abs + it.n_col - (uint64_t)i * group);
+    for (uint64_t h = h_lo; h < h_hi; h += hpm) f(i, (uint32_t)h, (uint32_t)std::min<uint64_t>(hpm, h_hi - h));
+  }
+}
+
+// The call as one unit launch (units.hip), when that is the faster way; false: as prefill units and
+// decode items.
+bool plan_units(const PlanIn& in, PlanOut& o) {
+  // explicit split settings address the prefill and decode kernels
+  if (!in.unit_w[0] || in.bt_shift < 4 || in.prefill_min_rows || in.decode_target_items || in.decode_min_tiles) return false;
+  const uint64_t group = in.n_head / in.n_kv;
+  if (group > 0xffff || in.n_kv > 0xffff) return false;   // a wave's record packs both
+  const bool f32 = in.kv_type == LMH_KV_F32, pf_ok = in.scale > 0.f && in.layout == LAYOUT_TILES && in.prefill_supported;
+  bool multi = false;
+  uint64_t max_pages = 0, steps16 = 0, steps32 = 0, steps_rows = 0;   // steps_*: 16-key tiles walked, per KV head
+  for (uint64_t i = 0; i < in.n_segs; i++) {
+    const lmh_seg& sg = in.segs[i];
+    if (sg.n == 0) continue;
+    if (pf_ok && sg.n >= DEFAULT_PREFILL_MIN_ROWS) return false;
+    multi |= sg.n > 1;
+    const uint64_t last = sg.pos0 + sg.n - 1;
+    const uint64_t pages = last / 16 - key_lo(sg.pos0, in.window) / 16 + 1;
+    max_pages = std::max(max_pages, last / 16 - key_lo(last, in.window) / 16 + 1);
+    steps_rows += sg.n * ((group + 15) / 16) * pages;
+    steps16 += (sg.n * group + 15) / 16 * pages;
+    steps32 += (sg.n * group + 31) / 32 * pages;
+  }
+  // Decode rows alone: the row layout's, and f32 pages' of wide groups (16 rows x 3,000 keys, hd 128:
+  // group 8 166.6 -> 103.0 us; group 4 113.0 -> 102.5 but 16 x 700 36.2 -> 37.2, group 1 77.9 -> 101.4).
+  if (!multi && in.layout == LAYOUT_TILES && !(f32 && group >= 8 && max_pages > 16)) return false;
+  // Short segments on the decode item's pages: when sharing the walks saves the device's waves ten
+  // tiles each or more (32/8 heads, hd 128, f16: 8 x 2 rows of 2,000 keys 20.4 -> 24.6 us, saves 8;
+  // 5 rows of 6,000 24.4 -> 20.3, saves 11; 32 x 3 of 700 43.2 -> 23.6, saves 22).
+  if (in.layout == LAYOUT_TILES && !f32 && (steps_rows - std::min(steps_rows, in.unit_w[1] ? steps32 : steps16)) * in.n_kv < 40ull * in.n_cu)
+    return false;
+  o.ng = (uint32_t)std::min<uint64_t>(group, 16);   // a partial slot holds the group's heads (pieces: group <= 16)
+  o.u_nb = in.unit_w[1] && 4 * steps32 < 3 * steps16 ? 2 : 1;
+  const uint32_t KT = f32 ? 1 : 2, cols = 16 * o.u_nb;
+  // A segment's column blocks; a unit is a block for one KV head.
+  struct Block {
+    PrefillItem it;
+    uint32_t ns;   // steps
+  };
+  std::vector<Block> blocks;
+  std::vector<uint32_t> seg0;   // each segment's first block
+  uint64_t total = 0, max_ns = 0;
+  for (uint64_t i = 0; i < in.n_segs; i++) {
+    const lmh_seg& sg = in.segs[i];
+    const uint64_t n_cols = sg.n * group;
+    seg0.push_back((uint32_t)blocks.size());
+    for (uint64_t c0 = 0; c0 < n_cols; c0 += cols) {
+      Block b{};
+      b.it.n_col = (uint32_t)std::min<uint64_t>(cols, n_cols - c0);
+      const uint64_t t0 = c0 / group, t1 = (c0 + b.it.n_col - 1) / group;
+      const uint64_t page_lo = key_lo(sg.pos0 + t0, in.window) / 16;
+      b.it.seq = (uint32_t)sg.seq;
+      b.it.row0 = (uint32_t)(sg.start + t0);
+      b.it.pos0 = (uint32_t)(sg.pos0 + t0);
+      b.it.n_tok = (uint32_t)(t1 - t0 + 1);
+      b.it.c_off = (uint32_t)(c0 % group);
+      b.it.page0 = (uint32_t)page_lo;
+      b.it.n_pages = (uint32_t)((sg.pos0 + t1) / 16 - page_lo + 1);
+      b.it.slot = NO_SLOT;
+      b.ns = (b.it.n_pages + KT - 1) / KT;
+      total += b.ns;
+      max_ns = std::max<uint64_t>(max_ns, b.ns);
+      blocks.push_back(b);
+    }
+  }
+  seg0.push_back((uint32_t)blocks.size());
+  total *= in.n_kv;
+  const uint64_t n_units = (uint64_t)blocks.size() * in.n_kv;
+  // Workgroups of the most waves share the longest units; where most units have a wave of their own
+  // anyway, smaller ones leave a CU's waves to finish and start independently.
+  const uint32_t w_max = in.unit_w[o.u_nb - 1], per_cu = std::max(in.unit_waves_per_cu[o.u_nb - 1], w_max);
+  const uint32_t W = 2 * n_units > (uint64_t)in.n_cu * per_cu ? std::min(4u, w_max) : w_max;
+  o.u_w = W;
+  const uint64_t wg_cap = (uint64_t)in.n_cu * (per_cu / W), target = wg_cap * W;
+  // More units than the device holds waves (or nearly, of very uneven lengths): several rounds.
+  // (hd 64 f32 prompts of 2,048 tokens, 2,048 units of 1 .. 128 steps: 207 us in rounds, 241 as one;
+  // hd 256 bf16 with a window, 850 units for 1,024 waves, lengths within 1.7 of the mean: 81, 67 us.)
+  const bool rounds = n_units > target || (2 * n_units > target && 5 * max_ns * n_units > 9 * total);
+  // Steps per wave c, a unit's waves ceil(steps / c), all resident at once: the smallest c whose
+  // waves fit if units may be cut into key pieces wherever a workgroup ends (c_cut; their partials
+  // merge in a launch of their own), and the smallest whose whole units pack into the workgroups
+  // (c_whole). Cutting has to save more than the merge launch costs.
+  const uint32_t c_min = 4 / KT;
+  const uint32_t slack = f32 ? 6 : 3;   // steps: the merge launch's ~4.5 us at ~1.5 us (a 16-key f32 step: 0.8 us)
+  const bool cut_ok = !in.prefill_no_split && !in.noalloc && group <= 16 && in.hdv <= 256 && in.hdv % 4 == 0;
+  auto smallest = [&](auto&& fits) {
+    uint32_t lo = (uint32_t)std::max<uint64_t>(c_min, (total + target - 1) / target), hi = std::max<uint32_t>(lo, (uint32_t)max_ns);
+    while (lo < hi) {
+      const uint32_t mid = (lo + hi) / 2;
+      if (fits(mid)) hi = mid;
+      else lo = mid + 1;
+    }
+    return lo;
+  };
+  uint32_t c;
+  bool cut = false;
+  if (rounds) {
+    c = (uint32_t)std::max<uint64_t>(c_min, (total + target - 1) / target);
+  } else {
+    const uint32_t c_cut = smallest([&](uint32_t x) {
+      uint64_t n = 0;
+      for (const Block& b : blocks) n += (b.ns + x - 1) / x;
+      return n * in.n_kv + W <= target;
+    });
+    const uint32_t c_whole = smallest([&](uint32_t x) {
+      uint64_t count[UNIT_MAX_WAVES + 1] = {}, wgs = 0;
+      for (const Block& b : blocks) {
+        const uint32_t n = (b.ns + x - 1) / x;
+        if (n > W) return false;
+        count[n] += in.n_kv;
+      }
+      for (uint32_t n = W; n >= 1; n--)   // best fit, longest first, over the counts
+        while (count[n]) {
+          uint32_t room = W;
+          for (uint32_t k = n; k >= 1; k--)
+            while (count[k] && k <= room) {
+              count[k]--;
+              room -= k;
+            }
+          wgs++;
+        }
+      return wgs <= wg_cap;
+    });
+    cut = cut_ok && c_whole > c_cut + slack;
+    c = cut ? c_cut : std::max(c_whole, (uint32_t)((max_ns + W - 1) / W));
+  }
+  // Members of workgroups: a unit, or a piece of one (whole 64-key tiles), with its waves.
+  struct Member {
+    uint32_t block, kvh, tile0, tile1, n, wg, at, piece;
+  };
+  std::vector<Member> mem;
+  mem.reserve(n_units + (cut ? wg_cap : 0));
+  auto pages_of = [&](const Member& m) {
+    const uint32_t n = blocks[m.block].it.n_pages;
+    return std::min(n, 4 * m.tile1) - 4 * m.tile0;
+  };
+  const uint32_t tile_steps = 4 / KT;
+  uint32_t n_wg = 0;
+  if (cut) {
+    // units in order, each workgroup filled before the next; a little longer waves where the cuts'
+    // rounding would take one workgroup too many
+    for (;; c++) {
+      mem.clear();
+      n_wg = 0;
+      uint32_t room = 0;
+      for (uint64_t i = 0; i < in.n_segs; i++)
+        for (uint32_t kvh = 0; kvh < in.n_kv; kvh++)
+          for (uint32_t b = seg0[i]; b < seg0[i + 1]; b++) {
+            const uint32_t tiles = (blocks[b].it.n_pages + 3) / 4;
+            uint32_t t = 0, piece = 0;
+            while (t < tiles) {
+              if (room == 0) {
+                n_wg++;
+                room = W;
+              }
+              const uint32_t rest = blocks[b].ns - t * tile_steps;
+              uint32_t n = (rest + c - 1) / c, t1 = tiles;
+              if (n > room) {   // what fits, unless that is next to nothing
+                const uint32_t take = std::max(1u, room * c / tile_steps);
+                if (take < 2 && n <= W) {
+                  room = 0;
+                  continue;
+                }
+                n = room;
+                t1 = piece + 1 == PF_MAX_PIECES ? tiles : std::min(tiles, t + take);
+              }
+              mem.push_back(Member{b, kvh, t, t1, n, n_wg - 1, W - room, piece++});
+              room -= n;
+              t = t1;
+            }
+          }
+      if (n_wg <= wg_cap || c >= max_ns) break;
+    }
+  } else {
+    // whole units, their waves capped at a workgroup's: those with the most waves first, so the
+    // workgroups fill; in rounds the longest waves first
+    for (uint64_t i = 0; i < in.n_segs; i++)
+      for (uint32_t kvh = 0; kvh < in.n_kv; kvh++)
+        for (uint32_t b = seg0[i]; b < seg0[i + 1]; b++)
+          mem.push_back(Member{b, kvh, 0, (blocks[b].it.n_pages + 3) / 4, std::min(W, (blocks[b].ns + c - 1) / c), 0, 0, 0});
+    auto key = [&](const Member& m) { return rounds ? (blocks[m.block].ns + m.n - 1) / m.n : m.n; };
+    std::vector<uint32_t> first((rounds ? (uint32_t)max_ns : W) + 2, 0);   // counting sort, largest key first
+    for (const Member& m : mem) first[key(m)]++;
+    uint32_t at = 0;
+    for (size_t k = first.size(); k-- > 0;) {
+      const uint32_t n = first[k];
+      first[k] = at;
+      at += n;
+    }
+    std::vector<Member> sorted(mem.size());
+    for (const Member& m : mem) sorted[first[key(m)]++] = m;
+    mem.swap(sorted);
+    std::vector<uint32_t> open[UNIT_MAX_WAVES + 1];   // workgroups by free waves
+    for (Member& m : mem) {
+      uint32_t f = m.n;
+      while (f <= W && open[f].empty()) f++;
+      if (f <= W) {
+        m.wg = open[f].back();
+        open[f].pop_back();
+      } else {
+        m.wg = n_wg++;
+        f = W;
+      }
+      m.at = W - f;
+      if (f > m.n) open[f - m.n].push_back(m.wg);
+    }
+  }
+  // Workgroup b runs on XCD b % 8: in one round, runs of consecutive workgroups go to one XCD, so
+  // units that read the same pages (a KV head's are consecutive) share its L2.
+  const uint32_t n_xcd = in.n_cu % 8 == 0 && !rounds ? 8 : 1, per_xcd = (n_wg + n_xcd - 1) / n_xcd;
+  auto launch_at = [&](uint32_t wg) { return n_xcd == 1 ? wg : wg % per_xcd * n_xcd + wg / per_xcd; };
+  // partial slots and merges of the units in several pieces (their members are consecutive), the heads
+  // of a merge few enough for about a thousand merge waves
+  uint64_t cut_cols = 0;
+  for (size_t i = 0; cut && i < mem.size(); i++) cut_cols += mem[i].piece == 1 ? blocks[mem[i].block].it.n_col : 0;
+  const uint32_t merge_heads = (uint32_t)std::max<uint64_t>(1, cut_cols / 1024);
+  o.uwaves.assign((size_t)per_xcd * n_xcd * W, UnitWave{});
+  std::vector<uint32_t> slots_of;   // per member: first slot of its unit
+  if (cut) slots_of.assign(mem.size(), NO_SLOT);
+  for (size_t i = 0; cut && i < mem.size();) {
+    size_t e = i + 1;
+    while (e < mem.size() && mem[e].piece != 0) e++;
+    const uint32_t k = (uint32_t)(e - i);
+    if (k > 1) {
+      const PrefillItem& it = blocks[mem[i].block].it;
+      const uint32_t base = o.slots, kvh = mem[i].kvh;
+      for (size_t x = i; x < e; x++) slots_of[x] = base;
+      for_each_merge(it, group, k, [&](uint32_t t, uint32_t h, uint32_t nh) {
+        o.merges.push_back(MergeItem{it.row0 + t, kvh, h, base + t * k, k, nh});
+      }, merge_heads);
+      o.slots += it.n_tok * k;
+      for (size_t x = i; x < e; x++) mem[x].piece |= k << 16;
+    }
+    i = e;
+  }
+  for (size_t i = 0; i < mem.size(); i++) {
+    const Member& m = mem[i];
+    const PrefillItem& it = blocks[m.block].it;
+    const uint32_t k = m.piece >> 16, n_pages = pages_of(m), page0 = it.page0 + 4 * m.tile0, ns = (n_pages + KT - 1) / KT;
+    const int32_t* tab = in.table + (uint64_t)it.seq * in.bps;
+    UnitWave* w = &o.uwaves[(size_t)launch_at(m.wg) * W + m.at];
+    const uint32_t n = std::min(m.n, ns);   // (a piece's waves each have a step)
+    for (uint32_t j = 0; j < n; j++) {
+      const uint32_t a = ns * j / n * KT, b = std::min(n_pages, ns * (j + 1) / n * KT);
+      const uint64_t p = page0 + a, p1 = std::min<uint64_t>(p + 1, page0 + b - 1);
+      w[j] = UnitWave{it.seq, it.row0, it.pos0, page0 + a, b - a, k ? slots_of[i] + (m.piece & 0xffffu) : NO_SLOT,
+                      {(uint32_t)tab[(p << 4) >> in.bt_shift], (uint32_t)tab[(p1 << 4) >> in.bt_shift]},
+                      m.kvh | it.c_off << 16, it.n_col | j << 8 | n << 16 | k << 24};
+    }
+    o.u_shared |= n > 1;
+  }
+  o.chunk = c * KT;
+  if (in.list_units) {   // as prefill units: pf_wg lists
+    std::vector<std::vector<uint32_t>> lists(n_wg);
+    for (uint32_t i = 0; i < mem.size(); i++) lists[mem[i].wg].push_back(i);
+    o.pf_wg = n_wg;
+    for (const auto& v : lists) o.pf_per_wg = std::max<uint32_t>(o.pf_per_wg, (uint32_t)v.size());
+    o.pitems.assign((size_t)o.pf_wg * o.pf_per_wg, PrefillItem{});
+    for (uint32_t b = 0; b < o.pf_wg; b++)
+      for (size_t j = 0; j < lists[b].size(); j++) {
+        const Member& m = mem[lists[b][j]];
+        PrefillItem it = blocks[m.block].it;
+        it.kvh = m.kvh;
+        it.n_pages = pages_of(m);
+        it.page0 += 4 * m.tile0;
+        if (m.piece >> 16) {
+          it.slot = slots_of[lists[b][j]] + (m.piece & 0xffffu);
+          it.slot_stride = m.piece >> 16;
+        }
+        const int32_t* tab = in.table + (uint64_t)it.seq * in.bps;
+        for (uint32_t e = 0; e < 8; e++)
+          it.blk[e] = (uint32_t)tab[((uint64_t)(it.page0 + std::min(e, it.n_pages - 1)) << 4) >> in.bt_shift];
+        o.max_pages = std::max(o.max_pages, it.n_pages);
+        o.pitems[(size_t)b * o.pf_per_wg + j] = it;
+      }
+  }
+  return true;
+}
+
 // Whole units grouped per workgroup, longest-processing-time-first: units by decreasing cost (ties
 // in list order), each to the currently least loaded workgroup (ties to the lower index). Returns
 // the largest workgroup load. The loads live in a binary min-heap of (load, workgroup) whose top
@@ -120,6 +412,10 @@ void plan_attend(const PlanIn& in, PlanOut& o) {
   o.pitems.clear();
   o.slots = o.pf_wg = o.pf_per_wg = o.max_pages = 0;
   o.local = 0;
+  o.uwaves.clear();
+  o.u_nb = o.u_w = 0;
+  o.u_shared = false;
+  if (plan_units(in, o)) return;
   auto blk_at = [&](uint64_t seq, uint64_t p) {   // block id of the tile holding key p
     return (uint32_t)in.table[seq * in.bps + (((p >> 4) << 4) >> in.bt_shift)];
   };
@@ -204,21 +500,9 @@ void plan_attend(const PlanIn& in, PlanOut& o) {
     const double cap = (w_cut + PF_UNIT_COST * ((double)units.size() + slots)) / std::max<uint32_t>(slots, 1);
     const bool try_cut = !in.prefill_no_split && group <= 16 && !units.empty() && max_tiles >= 2 * PF_MIN_PIECE &&
                          cap < PF_CUT_GAIN * whole;
-    // A cut unit's merges: per token over the unit's heads of that token, in groups of heads whose
-    // partial rows (heads x pieces) one merge wave loads at once. for_each_merge(u, k, f) calls
-    // f(token, first head, heads) for each.
-    auto for_each_merge = [&](const PfUnit& u, uint32_t k, auto&& f) {
-      const uint32_t hpm = std::max<uint32_t>(1, PF_MERGE_ROWS / k);
-      const uint64_t c_abs = u.it.c_off;   // the unit's first column, counted from its first token
-      for (uint32_t i = 0; i < u.it.n_tok; i++) {
-        const uint64_t h_lo = i == 0 ? c_abs : 0;
-        const uint64_t h_hi = std::min<uint64_t>(group, c_abs + u.it.n_col - (uint64_t)i * group);
-        for (uint64_t h = h_lo; h < h_hi; h += hpm) f(i, (uint32_t)h, (uint32_t)std::min<uint64_t>(hpm, h_hi - h));
-      }
-    };
     auto piece_merges = [&](const PfUnit& u, uint32_t k) {
       uint64_t n = 0;
-      for_each_merge(u, k, [&](uint32_t, uint32_t, uint32_t) { n++; });
+      for_each_merge(u.it, group, k, [&](uint32_t, uint32_t, uint32_t) { n++; });
       return n;
     };
     const size_t pf_slot_bytes = (size_t)ng * (in.hdv + 4) * 4;   // a slot holds the group's heads (ng = group)
@@ -228,7 +512,7 @@ void plan_attend(const PlanIn& in, PlanOut& o) {
       const uint32_t k = (uint32_t)pieces.size();
       const uint32_t base = o.slots;
       if (k > 1) {
-        for_each_merge(u, k, [&](uint32_t i, uint32_t h, uint32_t nh) {
+        for_each_merge(u.it, group, k, [&](uint32_t i, uint32_t h, uint32_t nh) {
           o.merges.push_back(MergeItem{u.it.row0 + i, u.it.kvh, h, base + i * k, k, nh});
         });
         o.slots += u.it.n_tok * k;

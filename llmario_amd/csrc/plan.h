@@ -48,6 +48,9 @@ struct PlanIn {
   uint32_t rows_max_heads = 4;      // query heads per item of the row-layout kernel
   bool local_merge_ok = false;      // f32 decode: split rows may merge inside their workgroup
   bool mfma_local_ok = false;       // matrix-core decode: the same, for rows split at most 4 ways
+  uint32_t unit_w[2] = {0, 0};      // most waves per workgroup of the unit launch of 16 / 32 columns (0: no instance)
+  uint32_t unit_waves_per_cu[2] = {8, 8};   // its waves a CU holds at once
+  bool list_units = false;          // list the unit launch's units in pitems too (lmh_plan_attend)
 };
 
 struct PlanOut {
@@ -60,6 +63,9 @@ struct PlanOut {
   uint32_t pf_wg = 0, pf_per_wg = 0, max_pages = 0;
   uint32_t chunk = 0;                 // decode split chunk (16-key tiles)
   uint32_t local = 0;                 // decode items merge inside workgroups of this many waves (0: no)
+  std::vector<UnitWave> uwaves;       // a unit launch (units.hip) instead of all of the above but the merges
+  uint32_t u_nb = 0, u_w = 0;         // its 16-column blocks per unit and waves per workgroup
+  bool u_shared = false;              // some unit is shared between waves
 };
 
 // Segments of at least this many rows run on the matrix-core prefill kernel by default (Metal's

@@ -82,4 +82,18 @@ struct PrefillItem {
   uint32_t blk[8];
 };
 
+// One wave of a unit launch (units.hip): up to 16 or 32 columns of one segment and KV head, as a
+// PrefillItem's, over key pages page0 .. page0 + n_pages - 1: this wave's share of the unit's pages.
+// slot: as a PrefillItem's. blk: the block ids of the wave's first two pages (the last repeated).
+// head: the KV head | c_off << 16. cols: n_col | the wave's index among the unit's waves << 8 | their
+// number << 16 (consecutive waves of one workgroup; 0: an idle wave) | slot_stride << 24.
+constexpr int UNIT_MAX_WAVES = 8;   // waves per workgroup, and waves a unit's keys are shared by
+struct UnitWave {
+  uint32_t seq, row0, pos0;
+  uint32_t page0, n_pages;
+  uint32_t slot;
+  uint32_t blk[2];
+  uint32_t head, cols;
+};
+
 }  // namespace lmh

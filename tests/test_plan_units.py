@@ -1,0 +1,77 @@
+"""Which calls lmh_attend's planner gives to the unit launch (units.hip) and which to the prefill and
+decode kernels, on the CPU, over the forms the rule tells apart: page type and width (an instance or
+none), layout, segment lengths, head group, block size, split settings. Every plan is also checked to
+cover each row's keys once (check_plan: attend's ranges, crates/engine/model/src/forward.rs:585-807);
+the GPU tests compare the two routes' outputs."""
+
+import pytest
+
+from test_plan import check_plan, contiguous_table, plan
+
+# kv, (n_head, n_kv, hd, hdv), block, prior, new, options, expected: "units", "items" (decode items
+# alone) or "prefill" (prefill units, beside decode items if the call has decode rows)
+FORMS = [
+    ("f16", (32, 8, 128, 128), 16, [2000] * 4, [6] * 4, {}, "units"),
+    ("f16", (32, 8, 128, 128), 16, [2000] * 4, [1] * 4, {}, "items"),        # decode rows alone
+    ("f16", (32, 8, 128, 128), 16, [100] * 4, [2] * 4, {}, "items"),         # too little to share
+    ("f16", (32, 8, 128, 128), 16, [2000] * 4, [6, 6, 6, 8], {}, "prefill"),   # one long segment
+    ("f16", (32, 8, 128, 128), 16, [2000] * 4, [6] * 4, {"prefill_min_rows": 8}, "items"),
+    ("f16", (32, 8, 128, 128), 16, [2000] * 4, [6] * 4, {"decode_min_tiles": 8}, "items"),
+    ("q8_0", (32, 8, 128, 128), 32, [2000] * 4, [6] * 4, {}, "units"),
+    ("bf16", (16, 4, 256, 256), 16, [500, 40], [200, 1], {}, "units"),       # no prefill instance
+    ("f16", (12, 4, 96, 96), 64, [0], [500], {}, "units"),
+    ("q8_0", (12, 4, 96, 96), 16, [100], [50], {}, "items"),                 # row layout, q8_0: no instance
+    ("f16", (32, 32, 80, 80), 16, [700], [1], {}, "units"),                  # row layout, decode rows too
+    ("bf16", (8, 2, 80, 80), 16, [15], [3], {}, "units"),
+    ("f16", (8, 2, 100, 100), 16, [300], [5], {}, "items"),                  # width not a multiple of 8
+    ("f16", (8, 2, 80, 80), 8, [300], [5], {}, "items"),                     # blocks under 16 positions
+    ("f16", (8, 1, 512, 512), 16, [300], [5], {}, "items"),                  # wider than any instance
+    ("f16", (16, 4, 64, 128), 16, [300], [1], {}, "units"),
+    ("f32", (8, 8, 64, 64), 16, [255], [1], {}, "items"),
+    ("f32", (8, 8, 64, 64), 16, [255], [2], {}, "units"),
+    ("f32", (64, 8, 128, 128), 16, [900], [1], {}, "units"),                 # wide group, long row
+    ("f32", (64, 8, 128, 128), 16, [200], [1], {}, "items"),
+    ("f32", (8, 2, 100, 100), 16, [300], [1], {}, "units"),
+    ("f32", (8, 2, 50, 50), 16, [300], [1], {}, "items"),                    # width not a multiple of 4
+]
+
+
+@pytest.mark.parametrize("window", [0, 333])
+@pytest.mark.parametrize("kv,geo,bt,prior,new,opt,want", FORMS,
+                         ids=[f"{f[0]}-{'x'.join(map(str, f[1]))}-bt{f[2]}-{'_'.join(map(str, f[4]))}" + ("-set" if f[5] else "")
+                              for f in FORMS])
+def test_route_and_cover(kv, geo, bt, prior, new, opt, want, window):
+    segs, start = [], 0
+    for s, (p, n) in enumerate(zip(prior, new)):
+        segs.append((s, start, n, p))
+        start += n
+    table = contiguous_table([p + n for p, n in zip(prior, new)], bt)
+    for n_cu in (256, 80, 12):
+        for noalloc in (False, True):
+            items, merges, units, c = plan(kv, *geo, bt, table, segs, window=window, n_cu=n_cu, noalloc=noalloc, **opt)
+            check_plan(kv, *geo, bt, table, segs, window, items, merges, units, c, noalloc=noalloc)
+            if n_cu != 256 or window:
+                continue
+            small_units = len(units) > 0 and int(units[:, 6].max()) <= 32
+            got = "items" if len(units) == 0 else "units" if small_units and len(items) == 0 else "prefill"
+            assert got == want, (got, len(items), len(units))
+            if noalloc and got == "units":   # no partials outside the workgroups
+                assert c.slots == 0 and len(merges) == 0
+
+
+def test_long_units_are_cut_and_short_ones_packed():
+    """One long context: its units run as key pieces that a merge launch combines; many short rows:
+    whole units, no merges, and no more workgroups than the device holds at once."""
+    geo = (64, 8, 128, 128)
+    table = contiguous_table([9007], 16)
+    segs = [(0, 0, 7, 9000)]
+    items, merges, units, c = plan("f16", *geo, 16, table, segs)
+    check_plan("f16", *geo, 16, table, segs, 0, items, merges, units, c)
+    assert c.slots > 0 and len(merges) > 0 and len(items) == 0
+    assert c.pf_wg <= 512   # 8 waves per CU: 256 workgroups of 8, or 512 of 4
+    prior, new = [700 + 3 * i for i in range(32)], [3] * 32
+    table = contiguous_table([p + 3 for p in prior], 16)
+    segs = [(i, 3 * i, 3, p) for i, p in enumerate(prior)]
+    items, merges, units, c = plan("f16", 32, 8, 128, 128, 16, table, segs)
+    check_plan("f16", 32, 8, 128, 128, 16, table, segs, 0, items, merges, units, c)
+    assert c.slots == 0 and len(merges) == 0 and len(items) == 0 and c.pf_wg <= 512
