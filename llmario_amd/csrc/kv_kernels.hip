@@ -528,13 +528,21 @@ __global__ void gather_encoded_kernel(PageGeom g, const int32_t* row_seq, const 
   gather_enc_side(g, sl, true, v + (size_t)row * v_row);
 }
 
-// ---- snapshots (KvCache::write_seq / read_seq, kv.rs:1030-1130): one layer's share of a
+// ---- snapshots (KvCache::write_seq / read_seq, kv.rs:1030-1130): a run of layers' share of a
 // sequence's blocks in the reference's block format. Snapshot block i is the sequence's block i;
 // inside it, the layer's K rows then V rows (ref_off + slot*k_row, ref_off + bt*k_row + slot*v_row)
 // in the row encoding. One workgroup per position of the covered blocks (every slot, written or
 // not, so the bytes equal the reference's block byte for byte).
+// Every kernel takes layers of one geometry that follow one another in the block as blockIdx.y,
+// `stride` bytes apart in the page block and in the snapshot's alike.
+__device__ inline void at_layer(PageGeom& g, uint64_t& ref_off, uint32_t stride) {
+  g.k_off += blockIdx.y * stride;
+  g.v_off += blockIdx.y * stride;
+  ref_off += (uint64_t)blockIdx.y * stride;
+}
 __global__ void snapshot_write_kernel(PageGeom g, uint32_t seq, uint32_t bt, uint64_t bb, uint64_t ref_off,
-                                      uint32_t k_row, uint32_t v_row, uint8_t* out) {
+                                      uint32_t k_row, uint32_t v_row, uint32_t stride, uint8_t* out) {
+  at_layer(g, ref_off, stride);
   const uint32_t p = blockIdx.x, bi = p / bt, j = p % bt;
   const Slot sl = locate(g, (int)seq, p);
   uint8_t* blk = out + (size_t)bi * bb + ref_off;
@@ -542,7 +550,8 @@ __global__ void snapshot_write_kernel(PageGeom g, uint32_t seq, uint32_t bt, uin
   gather_enc_side(g, sl, true, blk + (size_t)bt * k_row + (size_t)j * v_row);
 }
 __global__ void snapshot_read_kernel(PageGeom g, uint32_t seq, uint32_t bt, uint64_t bb, uint64_t ref_off,
-                                     uint32_t k_row, uint32_t v_row, const uint8_t* in) {
+                                     uint32_t k_row, uint32_t v_row, uint32_t stride, const uint8_t* in) {
+  at_layer(g, ref_off, stride);
   const uint32_t p = blockIdx.x, bi = p / bt, j = p % bt;
   const Slot sl = locate(g, (int)seq, p);
   const uint8_t* blk = in + (size_t)bi * bb + ref_off;
@@ -968,6 +977,7 @@ struct SnapGeom {
   uint32_t seq, bt, k_row, v_row;
   uint64_t bb, ref_off;
   uint32_t seg_k, seg_v;  // bytes of one head's values in a K / V row of the reference encoding
+  uint32_t stride;        // bytes from one layer (blockIdx.y) to the next
 };
 // byte u of one head's segment of a row (token m) in the reference encoding, as a byte of the
 // staged page tile: element bytes for f16/bf16/f32, code or scale bytes for q8_0
@@ -987,6 +997,7 @@ __device__ inline uint32_t seg_to_tile(uint32_t type, bool is_v, uint32_t m, uin
 template <bool WRITE>
 __global__ __launch_bounds__(256) void snapshot_tiles_kernel(PageGeom g, SnapGeom sg, uint8_t* snap) {
   extern __shared__ __attribute__((aligned(16))) uint8_t smem[];
+  at_layer(g, sg.ref_off, sg.stride);
   const uint32_t tid = threadIdx.x;
   uint32_t id = blockIdx.x;
   const bool is_v = id & 1u;
@@ -1094,18 +1105,6 @@ __device__ inline void snapshot_side(const PageGeom& g, const SnapGeom& sg, uint
     stage16(span / 16, [&](uint32_t i) -> const uint8_t* { return rows + (size_t)i * 16; },
             [&](uint32_t i) -> uint8_t* { return rw_l + (size_t)i * 16; });
   };
-  // page byte of (token m, byte u of a head's row segment), relative to the head's staged bytes
-  auto page_byte = [&](uint32_t m, uint32_t u) -> uint32_t {
-    if constexpr (TYPE == KV_Q8) {
-      const uint32_t b = u / 34u, r = u % 34u;
-      if (r < 2) return TB + (m * (DIM / 32) + b) * 2u + r;
-      return elem_off(KV_Q8, is_v, m, 32u * b + r - 2u, DIM);
-    } else if constexpr (TYPE == KV_F32) {
-      return elem_off(KV_F32, is_v, m, u >> 2, DIM) + (u & 3u);
-    } else {
-      return elem_off(TYPE, is_v, m, u >> 1, DIM) + (u & 1u);
-    }
-  };
   if constexpr (TYPE == KV_Q8) {
     // whole q8_0 row blocks ([f16 scale][32 codes], 34 bytes, 2-byte aligned in the row run):
     // K codes of a block are 4 runs of 8 bytes in the tile; V codes hold 4 tokens per 4-byte
@@ -1193,66 +1192,119 @@ __device__ inline void snapshot_side(const PageGeom& g, const SnapGeom& sg, uint
     }
     return;
   }
+  // f16 / bf16: granules of 8 dims (16 bytes of a row). A K granule is one operand row of the tile; V
+  // granules go four tokens at a time, eight 8-byte runs (4 tokens of one dim) to or from four rows
+  // (8 layers x 4,000 tokens per direction: 226 us by bytes in eight launches, 165 in one, 53 so).
+  constexpr uint32_t NG = DIM / 8;   // granules of a head's row
+  auto pick = [](uint32_t a, uint32_t b, uint32_t sel) { return __builtin_amdgcn_perm(b, a, sel); };
+  auto rows4 = [&](const uint2 (&d)[8], uint4 (&r)[4]) {   // d[i]: 4 tokens of dim i -> r[k]: 8 dims of token k
+#pragma unroll
+    for (int k = 0; k < 4; k++) {
+      const uint32_t sel = (k & 1) ? 0x07060302u : 0x05040100u;
+      uint32_t w[4];
+#pragma unroll
+      for (int i = 0; i < 4; i++) w[i] = k < 2 ? pick(d[2 * i].x, d[2 * i + 1].x, sel) : pick(d[2 * i].y, d[2 * i + 1].y, sel);
+      r[k] = make_uint4(w[0], w[1], w[2], w[3]);
+    }
+  };
+  auto dims8 = [&](const uint4 (&r)[4], uint2 (&d)[8]) {   // the inverse
+#pragma unroll
+    for (int i = 0; i < 8; i++) {
+      const uint32_t sel = (i & 1) ? 0x07060302u : 0x05040100u;
+      const uint32_t w0 = ((const uint32_t*)&r[0])[i >> 1], w1 = ((const uint32_t*)&r[1])[i >> 1];
+      const uint32_t w2 = ((const uint32_t*)&r[2])[i >> 1], w3 = ((const uint32_t*)&r[3])[i >> 1];
+      d[i] = make_uint2(pick(w0, w1, sel), pick(w2, w3, sel));
+    }
+  };
   if (WRITE) {
     stage_page();
     __syncthreads();
-    for (uint32_t c = tid; c < span / 16; c += 256) {
-      const uint32_t x0 = c * 16;
-      uint32_t m = x0 / row, rem = x0 - m * row, h = rem / SEG, u = rem - h * SEG;
-      uint32_t w4[4];
-#pragma unroll
-      for (int k = 0; k < 4; k++) {
-        uint32_t acc = 0;
-#pragma unroll
-        for (int j = 0; j < 4; j++) {
-          acc |= (uint32_t)pg_l[h * PH + page_byte(m, u)] << (8 * j);
-          if (++u == SEG) {
-            u = 0;
-            if (++h == nkv) {
-              h = 0;
-              m++;
-            }
-          }
-        }
-        w4[k] = acc;
+    if constexpr (!IS_V) {
+      for (uint32_t c = tid; c < 16 * nkv * NG; c += 256) {
+        const uint32_t m = c / (nkv * NG), rem = c - m * (nkv * NG), h = rem / NG, gi = rem - h * NG;
+        *(uint4*)(rows + (size_t)c * 16) = *(const uint4*)(pg_l + h * PH + k16_off(m, 8 * gi));
       }
-      *(uint4*)(rows + x0) = make_uint4(w4[0], w4[1], w4[2], w4[3]);
+    } else {
+      for (uint32_t c = tid; c < 4 * nkv * NG; c += 256) {
+        const uint32_t qg = c / (nkv * NG), rem = c - qg * (nkv * NG), h = rem / NG, gi = rem - h * NG;
+        uint2 d[8];
+        uint4 r[4];
+#pragma unroll
+        for (int i = 0; i < 8; i++) d[i] = *(const uint2*)(pg_l + h * PH + v16_off(4 * qg, 8 * gi + i));
+        rows4(d, r);
+#pragma unroll
+        for (int k = 0; k < 4; k++) *(uint4*)(rows + (size_t)(4 * qg + k) * row + rem * 16) = r[k];
+      }
     }
   } else {
     stage_rows();
     __syncthreads();
-    for (uint32_t c = tid; c < span / 16; c += 256) {
-      const uint32_t x0 = c * 16;
-      uint32_t m = x0 / row, rem = x0 - m * row, h = rem / SEG, u = rem - h * SEG;
-#pragma unroll
-      for (int j = 0; j < 16; j++) {
-        pg_l[h * PH + page_byte(m, u)] = rw_l[x0 + j];
-        if (++u == SEG) {
-          u = 0;
-          if (++h == nkv) {
-            h = 0;
-            m++;
-          }
-        }
+    if constexpr (!IS_V) {
+      for (uint32_t c = tid; c < 16 * nkv * NG; c += 256) {   // page order: 16 keys of a granule are 256 bytes
+        const uint32_t h = c / (16 * NG), rem = c - h * (16 * NG);
+        const uint32_t m = rem & 15u, gi = rem >> 4;
+        *(uint4*)(head0 + (size_t)h * sd.head + t * TB + rem * 16) = *(const uint4*)(rw_l + m * row + h * SEG + gi * 16);
       }
-    }
-    __syncthreads();
-    for (uint32_t h = 0; h < nkv; h++) {
-      uint8_t* dst = head0 + (size_t)h * sd.head;
-      for (uint32_t o = tid * 16; o < TB; o += 256 * 16) *(uint4*)(dst + t * TB + o) = *(const uint4*)(pg_l + h * PH + o);
-      if constexpr (TS > 0)
-        for (uint32_t o = tid * 4; o < TS; o += 256 * 4)
-          *(uint32_t*)(dst + sd.scale + t * TS + o) = *(const uint32_t*)(pg_l + h * PH + TB + o);
+    } else {
+      for (uint32_t c = tid; c < 4 * nkv * NG; c += 256) {
+        const uint32_t qg = c / (nkv * NG), rem = c - qg * (nkv * NG), h = rem / NG, gi = rem - h * NG;
+        uint2 d[8];
+        uint4 r[4];
+#pragma unroll
+        for (int k = 0; k < 4; k++) r[k] = *(const uint4*)(rw_l + (4 * qg + k) * row + rem * 16);
+        dims8(r, d);
+#pragma unroll
+        for (int i = 0; i < 8; i++) *(uint2*)(pg_l + h * PH + v16_off(4 * qg, 8 * gi + i)) = d[i];
+      }
+      __syncthreads();
+      for (uint32_t c = tid; c < nkv * TB / 16; c += 256) {
+        const uint32_t h = c / (TB / 16), o = (c - h * (TB / 16)) * 16;
+        *(uint4*)(head0 + (size_t)h * sd.head + t * TB + o) = *(const uint4*)(pg_l + h * PH + o);
+      }
     }
   }
 }
 template <bool WRITE, int TYPE, int DIM>
 __global__ __launch_bounds__(256) void snapshot_side_kernel(PageGeom g, SnapGeom sg, uint8_t* snap) {
   extern __shared__ __attribute__((aligned(16))) uint8_t smem[];
+  at_layer(g, sg.ref_off, sg.stride);
   if (blockIdx.x & 1u)
     snapshot_side<WRITE, TYPE, DIM, true>(g, sg, snap, smem);
   else
     snapshot_side<WRITE, TYPE, DIM, false>(g, sg, snap, smem);
+}
+
+// Pages that hold a head's rows as the snapshot does (f32 tiles; 16-bit and f32 row layout): a copy of
+// segments, in words of 16 or 4 bytes. One workgroup per 2,048 words of one block's K or V rows (z: the
+// side), eight words in flight per thread.
+template <bool WRITE, typename W>
+__global__ __launch_bounds__(256) void snapshot_copy_kernel(PageGeom g, SnapGeom sg, uint32_t parts, uint8_t* snap) {
+  at_layer(g, sg.ref_off, sg.stride);
+  const bool is_v = blockIdx.z != 0;
+  const Side sd = side(g, is_v);
+  const uint32_t bi = blockIdx.x / parts, part = blockIdx.x - bi * parts;
+  const uint32_t row = is_v ? sg.v_row : sg.k_row, seg = is_v ? sg.seg_v : sg.seg_k;
+  const uint32_t n = sg.bt * row / sizeof(W), rows_w = row / sizeof(W), seg_w = seg / sizeof(W);
+  const int blk = g.table[(size_t)sg.seq * g.bps + bi];
+  uint8_t* page = g.pool + (size_t)blk * g.block_bytes + sd.off;
+  W* rows = (W*)(snap + (size_t)bi * sg.bb + sg.ref_off + (is_v ? (size_t)sg.bt * sg.k_row : 0));
+  const uint32_t rpt = min(sg.bt, 16u);   // rows of a tile
+  auto at = [&](uint32_t i) -> W* {       // word i of the block's rows, in the page
+    const uint32_t j = i / rows_w, u = i - j * rows_w, h = u / seg_w, e = u - h * seg_w;
+    return (W*)(page + (size_t)h * sd.head + (j / rpt) * sd.tile + (j % rpt) * seg) + e;
+  };
+  const uint32_t base = part * 2048 + threadIdx.x;
+  W v[8];
+#pragma unroll
+  for (uint32_t k = 0; k < 8; k++) {
+    const uint32_t i = min(base + k * 256, n - 1);   // past the end: the last word again, not stored
+    v[k] = WRITE ? *at(i) : rows[i];
+  }
+#pragma unroll
+  for (uint32_t k = 0; k < 8; k++) {
+    const uint32_t i = base + k * 256;
+    if (i < n) *(WRITE ? rows + i : at(i)) = v[k];
+  }
 }
 
 // Zero whole blocks (a newly backed block reads as zeros, like the reference's anonymous
@@ -1380,13 +1432,14 @@ hipError_t launch_qk_rope_store(const PageGeom& g, const RopeGeom& r, const int3
 }
 
 hipError_t launch_snapshot(bool write, const PageGeom& g, uint32_t seq, uint32_t n_pos, uint32_t bt, uint64_t bb,
-                           uint64_t ref_off, uint32_t k_row, uint32_t v_row, uint8_t* bytes, hipStream_t s) {
-  if (n_pos == 0) return hipSuccess;
+                           uint64_t ref_off, uint32_t k_row, uint32_t v_row, uint32_t n_layers, uint8_t* bytes, hipStream_t s) {
+  if (n_pos == 0 || n_layers == 0) return hipSuccess;
   const uint32_t seg_k = k_row / g.n_kv, seg_v = v_row / g.n_kv;
   const bool tiles = g.layout == LAYOUT_TILES;
+  const uint32_t stride = bt * (k_row + v_row);   // a layer's bytes of a block, page and snapshot alike
   if (tiles && g.hd == g.hdv && bt % 16 == 0 && (g.kv_type == KV_F16 || g.kv_type == KV_BF16 || g.kv_type == KV_Q8) &&
       (g.hd == 64 || g.hd == 128 || g.hd == 256)) {
-    const SnapGeom sg{seq, bt, k_row, v_row, bb, ref_off, seg_k, seg_v};
+    const SnapGeom sg{seq, bt, k_row, v_row, bb, ref_off, seg_k, seg_v, stride};
     const uint32_t ph = g.k_tile + (g.kv_type == KV_Q8 ? g.k_tile_s : 0);
     const size_t lds = ((g.n_kv * ph + 15) & ~15u) + (write && g.kv_type != KV_Q8 ? 0 : 16 * (size_t)k_row);
     if (lds <= 64 * 1024) {
@@ -1394,9 +1447,9 @@ hipError_t launch_snapshot(bool write, const PageGeom& g, uint32_t seq, uint32_t
 #define LMH_SNAP(T, D)                                                                                       \
   if (g.kv_type == T && g.hd == D) {                                                                          \
     if (write)                                                                                                \
-      hipLaunchKernelGGL((snapshot_side_kernel<true, T, D>), dim3(n_wg), dim3(256), lds, s, g, sg, bytes);    \
+      hipLaunchKernelGGL((snapshot_side_kernel<true, T, D>), dim3(n_wg, n_layers), dim3(256), lds, s, g, sg, bytes);    \
     else                                                                                                      \
-      hipLaunchKernelGGL((snapshot_side_kernel<false, T, D>), dim3(n_wg), dim3(256), lds, s, g, sg, bytes);   \
+      hipLaunchKernelGGL((snapshot_side_kernel<false, T, D>), dim3(n_wg, n_layers), dim3(256), lds, s, g, sg, bytes);   \
     return hipGetLastError();                                                                                 \
   }
       LMH_SNAP(KV_F16, 64) LMH_SNAP(KV_F16, 128) LMH_SNAP(KV_F16, 256)
@@ -1405,23 +1458,36 @@ hipError_t launch_snapshot(bool write, const PageGeom& g, uint32_t seq, uint32_t
 #undef LMH_SNAP
     }
   }
+  if ((g.kv_type == KV_F32 || (!tiles && g.kv_type != KV_Q8)) && seg_k % 4 == 0 && seg_v % 4 == 0 &&
+      stride % 4 == 0 && bb % 4 == 0 && ((uintptr_t)bytes & 3) == 0) {
+    const SnapGeom sg{seq, bt, k_row, v_row, bb, ref_off, seg_k, seg_v, stride};
+    const bool wide = seg_k % 16 == 0 && seg_v % 16 == 0 && bb % 16 == 0 && ref_off % 16 == 0 && ((uintptr_t)bytes & 15) == 0;
+    const uint32_t words = bt * std::max(k_row, v_row) / (wide ? 16 : 4), parts = (words + 2047) / 2048;
+    const dim3 grid(n_pos / bt * parts, n_layers, 2);
+    if (wide && write) hipLaunchKernelGGL((snapshot_copy_kernel<true, uint4>), grid, dim3(256), 0, s, g, sg, parts, bytes);
+    else if (wide) hipLaunchKernelGGL((snapshot_copy_kernel<false, uint4>), grid, dim3(256), 0, s, g, sg, parts, bytes);
+    else if (write) hipLaunchKernelGGL((snapshot_copy_kernel<true, uint32_t>), grid, dim3(256), 0, s, g, sg, parts, bytes);
+    else hipLaunchKernelGGL((snapshot_copy_kernel<false, uint32_t>), grid, dim3(256), 0, s, g, sg, parts, bytes);
+    return hipGetLastError();
+  }
   if (tiles && seg_k % 4 == 0 && seg_v % 4 == 0 && bt % 16 == 0) {
-    const SnapGeom sg{seq, bt, k_row, v_row, bb, ref_off, seg_k, seg_v};
+    const SnapGeom sg{seq, bt, k_row, v_row, bb, ref_off, seg_k, seg_v, stride};
     const uint32_t tb = std::max(g.k_tile + (g.kv_type == KV_Q8 ? g.k_tile_s : 0),
                                  g.v_tile + (g.kv_type == KV_Q8 ? g.v_tile_s : 0));
     const size_t lds = ((tb + 15) & ~15u) + 16 * (size_t)std::max(seg_k, seg_v);
     const uint32_t n_wg = n_pos / 16 * g.n_kv * 2;
     if (write)
-      hipLaunchKernelGGL(snapshot_tiles_kernel<true>, dim3(n_wg), dim3(256), lds, s, g, sg, bytes);
+      hipLaunchKernelGGL(snapshot_tiles_kernel<true>, dim3(n_wg, n_layers), dim3(256), lds, s, g, sg, bytes);
     else
-      hipLaunchKernelGGL(snapshot_tiles_kernel<false>, dim3(n_wg), dim3(256), lds, s, g, sg, bytes);
+      hipLaunchKernelGGL(snapshot_tiles_kernel<false>, dim3(n_wg, n_layers), dim3(256), lds, s, g, sg, bytes);
     return hipGetLastError();
   }
   if (write)
-    hipLaunchKernelGGL(snapshot_write_kernel, dim3(n_pos), dim3(256), 0, s, g, seq, bt, bb, ref_off, k_row, v_row, bytes);
+    hipLaunchKernelGGL(snapshot_write_kernel, dim3(n_pos, n_layers), dim3(256), 0, s, g, seq, bt, bb, ref_off, k_row, v_row,
+                       stride, bytes);
   else
-    hipLaunchKernelGGL(snapshot_read_kernel, dim3(n_pos), dim3(256), 0, s, g, seq, bt, bb, ref_off, k_row, v_row,
-                       (const uint8_t*)bytes);
+    hipLaunchKernelGGL(snapshot_read_kernel, dim3(n_pos, n_layers), dim3(256), 0, s, g, seq, bt, bb, ref_off, k_row, v_row,
+                       stride, (const uint8_t*)bytes);
   return hipGetLastError();
 }
 
