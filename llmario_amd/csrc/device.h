@@ -108,6 +108,11 @@ struct RopeGeom {
   const float* freq_div;  // [half_rot] or null
   const float* freq;      // [half_rot] theta^(-2i/rot_dim), computed on the host
 };
+// One row (or the first of an aligned run of four) of a fused store, as the host stages it: a kernel
+// that has it needs no further look-up before its loads.
+struct RopeRow {
+  uint32_t row, pos, blk, pad;   // stacked row, position, block id
+};
 constexpr uint32_t ROPE_Q_NORM = 1, ROPE_K_NORM = 2, ROPE_V_NORM = 4, ROPE_APPLY = 8, ROPE_NEOX = 16;
 constexpr uint32_t ROPE_MAX_DIM = 512;  // largest hd / hdv the fused kernel stages per wave
 
@@ -139,7 +144,7 @@ hipError_t launch_gather_encoded(const PageGeom& g, const int32_t* row_seq, cons
                                  hipStream_t s);
 hipError_t launch_qk_rope_store(const PageGeom& g, const RopeGeom& r, const int32_t* row_seq, const int32_t* row_pos,
                                 uint32_t n_rows, const float* q, const float* k, const float* v, float* q_out,
-                                const int32_t* quads, uint32_t n_quads, const int32_t* rest, uint32_t n_rest,
+                                const RopeRow* quads, uint32_t n_quads, const RopeRow* rest, uint32_t n_rest,
                                 hipStream_t s, const LaunchEv& ev = {});
 // The share of n_layers layers of one geometry, consecutive in the block, of a sequence's snapshot
 // (write: pages -> reference block format; read: the reverse), positions 0 .. n_pos-1.

@@ -1366,31 +1366,30 @@ int32_t lmh_qk_rope_store(lmh_kv* kv, uint32_t layer, const lmh_seg* segs, uint6
   const int32_t *rs, *rp;
   const uint8_t* ex;
   int slot;
-  // rows of f16 / bf16 segments in aligned runs of 4 positions go to the 4-token kernel (whole
-  // 8-byte V runs); the others (decode rows, segment edges) to the per-row kernel
-  std::vector<int32_t> lists;  // [quads..., rest...]
+  // rows in aligned runs of 4 positions go to the 4-token kernel (whole words of a V tile); the others
+  // (decode rows, segment edges) to the per-row kernel
+  std::vector<RopeRow> lists;  // [quads..., rest...]
   uint32_t n_quads = 0;
-  if (kv->kv_type == LMH_KV_F16 || kv->kv_type == LMH_KV_BF16) {
-    std::vector<int32_t> rest;
+  if (y.layout == LAYOUT_TILES) {
+    const std::vector<int32_t>& tab = y.win ? kv->h_wtable : kv->h_table;
+    std::vector<RopeRow> rest;
     for (uint64_t i = 0; i < n_segs; i++) {
       const lmh_seg& sg = segs[i];
       for (uint64_t j = 0; j < sg.n;) {
-        if (((sg.pos0 + j) & 3) == 0 && j + 4 <= sg.n) {
-          lists.push_back((int32_t)(sg.start + j));
-          j += 4;
-        } else {
-          rest.push_back((int32_t)(sg.start + j));
-          j++;
-        }
+        const uint64_t pos = sg.pos0 + j;
+        const RopeRow row{(uint32_t)(sg.start + j), (uint32_t)pos, (uint32_t)tab[sg.seq * kv->bps + (pos >> kv->bt_shift)], 0};
+        const bool run = (pos & 3) == 0 && j + 4 <= sg.n;
+        (run ? lists : rest).push_back(row);
+        j += run ? 4 : 1;
       }
     }
     n_quads = (uint32_t)lists.size();
     lists.insert(lists.end(), rest.begin(), rest.end());
   }
   const size_t freq_bytes = freq.size() * 4;
-  if ((rc = kv->stage_rows(freq.data(), freq_bytes, lists.data(), lists.size() * 4, rs, rp, ex, slot)) != LMH_OK)
+  if ((rc = kv->stage_rows(freq.data(), freq_bytes, lists.data(), lists.size() * sizeof(RopeRow), rs, rp, ex, slot)) != LMH_OK)
     return rc;
-  const int32_t* d_lists = (const int32_t*)(ex + (freq_bytes + 255) / 256 * 256);
+  const RopeRow* d_lists = (const RopeRow*)(ex + (freq_bytes + 255) / 256 * 256);
   RopeGeom r{y.n_head, q_stride, p->flags, half_rot, p->eps, p->freq_scale, p->attn_factor,
              (p->flags & LMH_ROPE_Q_NORM) ? p->q_norm : nullptr, (p->flags & LMH_ROPE_K_NORM) ? p->k_norm : nullptr,
              apply ? p->freq_div : nullptr, (const float*)ex};

@@ -38,6 +38,12 @@ __device__ inline Slot locate(const PageGeom& g, int seq, uint32_t pos) {
   return s;
 }
 
+// The same for a listed row, whose block the host looked up.
+__device__ inline Slot locate(const PageGeom& g, const RopeRow& r) {
+  const uint32_t in_blk = r.pos & ((1u << g.bt_shift) - 1u);
+  return Slot{g.pool + (size_t)r.blk * g.block_bytes, in_blk >> 4, in_blk & 15u};
+}
+
 // f32 -> f16, round to nearest even (v_cvt_f16_f32 under the default rounding mode).
 __device__ inline uint16_t f16_bits(float x) {
   _Float16 h = (_Float16)x;
@@ -573,15 +579,14 @@ __global__ void snapshot_read_kernel(PageGeom g, uint32_t seq, uint32_t bt, uint
 // (a decode row or a chunk's unaligned edge), V written per element as in the row kernel.
 // Items it0 .. n_items-1 of [Q heads][K heads][V heads] are the workgroup's share.
 template <int VPL, int NT>
-__device__ void rope_tokens(const PageGeom& g, const RopeGeom& r, float2 (*cs)[ROPE_MAX_DIM / 2], uint32_t row0,
-                            uint32_t it0, uint32_t n_items, const int32_t* row_seq, const int32_t* row_pos,
-                            const float* q, const float* k, const float* v, float* q_out) {
+__device__ void rope_tokens(const PageGeom& g, const RopeGeom& r, float2 (*cs)[ROPE_MAX_DIM / 2], const RopeRow& rr,
+                            uint32_t it0, uint32_t n_items, const float* q, const float* k, const float* v, float* q_out) {
   constexpr uint32_t HD = 64 * VPL;
   constexpr int GRP = 2;  // heads (x 4 tokens) a wave requests before processing them (more heads
                           // cost occupancy: 2 keeps the kernel at 4 waves per SIMD)
   typedef float fv __attribute__((ext_vector_type(VPL)));
   const uint32_t tid = threadIdx.x, w = tid >> 6, lane = tid & 63u;
-  const uint32_t pos0 = (uint32_t)row_pos[row0];
+  const uint32_t row0 = rr.row, pos0 = rr.pos;
   auto src_of = [&](uint32_t it, uint32_t t) -> const float* {
     const size_t row = row0 + t;
     if (it < r.n_head) return q + (row * r.n_head + it) * r.q_stride;
@@ -604,7 +609,7 @@ __device__ void rope_tokens(const PageGeom& g, const RopeGeom& r, float2 (*cs)[R
     sincosf(angle, &sn, &cn);
     cs[t][ii] = make_float2(cn * r.attn_factor, sn * r.attn_factor);
   }
-  const Slot sl0 = locate(g, row_seq[row0], pos0);
+  const Slot sl0 = locate(g, rr);
   fv wq, wk;
 #pragma unroll
   for (int c = 0; c < VPL; c++) {
@@ -704,19 +709,26 @@ __device__ void rope_tokens(const PageGeom& g, const RopeGeom& r, float2 (*cs)[R
 // list), in one launch. blockIdx.y picks the workgroup's share of the heads, items y*ipw .. y*ipw+ipw-1, so a
 // short call still spreads over the chip instead of leaving each workgroup a long chain of round
 // trips.
+// Row x of the single rows: those of the runs taken apart (4 per run), then the rest.
+__device__ inline RopeRow single_row(const RopeRow* quads, uint32_t n_apart, const RopeRow* rest, uint32_t x) {
+  if (x >= 4 * n_apart) return rest[x - 4 * n_apart];
+  RopeRow r = quads[x >> 2];
+  r.row += x & 3u;
+  r.pos += x & 3u;   // a run lies in one tile
+  return r;
+}
+
 template <int VPL>
-__global__ __launch_bounds__(256) void qk_rope_store_quad_kernel(PageGeom g, RopeGeom r, const int32_t* quads,
-                                                                 uint32_t n_quads, const int32_t* rest,
-                                                                 const int32_t* row_seq, const int32_t* row_pos,
+__global__ __launch_bounds__(256) void qk_rope_store_quad_kernel(PageGeom g, RopeGeom r, const RopeRow* quads,
+                                                                 uint32_t n_quads, uint32_t n_apart, const RopeRow* rest,
                                                                  const float* q, const float* k, const float* v,
                                                                  float* q_out, uint32_t ipw) {
   __shared__ float2 cs[4][ROPE_MAX_DIM / 2];
   const uint32_t it0 = blockIdx.y * ipw, n_items = min(r.n_head + 2 * g.n_kv, it0 + ipw);
   if (blockIdx.x < n_quads)
-    rope_tokens<VPL, 4>(g, r, cs, (uint32_t)quads[blockIdx.x], it0, n_items, row_seq, row_pos, q, k, v, q_out);
+    rope_tokens<VPL, 4>(g, r, cs, quads[blockIdx.x], it0, n_items, q, k, v, q_out);
   else
-    rope_tokens<VPL, 1>(g, r, cs, rest ? (uint32_t)rest[blockIdx.x - n_quads] : blockIdx.x - n_quads, it0, n_items,
-                        row_seq, row_pos, q, k, v, q_out);
+    rope_tokens<VPL, 1>(g, r, cs, single_row(quads, n_apart, rest, blockIdx.x - n_quads), it0, n_items, q, k, v, q_out);
 }
 
 // Sum over each group of 8 lanes, the same bits in all 8 (DPP: lane l + lane 7-l, then the quad
@@ -726,6 +738,26 @@ __device__ inline float lanes8_sum(float s) {
   s += __builtin_amdgcn_update_dpp(0.f, s, 0xb1, 0xf, 0xf, false);   // quad_perm [1,0,3,2]
   s += __builtin_amdgcn_update_dpp(0.f, s, 0x4e, 0xf, 0xf, false);   // quad_perm [2,3,0,1]
   return s;
+}
+// Max over each group of 8 lanes, and of 4, 8 or 16 (the same value in all of them).
+__device__ inline float lanes4_max(float s) {
+  s = fmaxf(s, __builtin_amdgcn_update_dpp(0.f, s, 0xb1, 0xf, 0xf, false));
+  return fmaxf(s, __builtin_amdgcn_update_dpp(0.f, s, 0x4e, 0xf, 0xf, false));
+}
+__device__ inline float lanes8_max(float s) {
+  return lanes4_max(fmaxf(s, __builtin_amdgcn_update_dpp(0.f, s, 0x141, 0xf, 0xf, false)));
+}
+template <int N>
+__device__ inline float lanes_max(float s) {
+  static_assert(N == 4 || N == 8 || N == 16, "lanes of a block");
+  if constexpr (N == 16) s = fmaxf(s, __builtin_amdgcn_update_dpp(0.f, s, 0x140, 0xf, 0xf, false));
+  if constexpr (N >= 8) return lanes8_max(s);
+  return lanes4_max(s);
+}
+// Four q8_0 codes (quantize_q8_0, kv.rs:156-171: round to nearest even of x * id) packed in a word.
+__device__ inline uint32_t q8x4(float a, float b, float c, float d, float id) {
+  auto q = [&](float x) { return (uint32_t)(uint8_t)(int8_t)(int32_t)rintf(x * id); };
+  return q(a) | q(b) << 8 | q(c) << 16 | q(d) << 24;
 }
 // Sum over each half wave (32 lanes), the same bits in all of them.
 __device__ inline float lanes32_sum(float s) {
@@ -747,7 +779,7 @@ __device__ inline uint32_t pack16x2(float a, float b) {
   }
 }
 
-// An aligned run of 4 f16 / bf16 tokens when hd == hdv == HD (64, 128, 256) and every rotated
+// An aligned run of 4 tokens when hd == hdv == HD (64, 128, 256) and every rotated
 // pair sits in one lane (Normal pairs; Neox over all HD dims): the same results as
 // rope_tokens<HD / 64, 4>, with the work counted in slots of two heads of one kind (Q, K or V) for
 // the run's four tokens, so every lane of a wave runs the same code, and every access 8 or 16
@@ -758,17 +790,22 @@ __device__ inline uint32_t pack16x2(float a, float b) {
 //   and each float4 of K is half of one 16-byte operand row of the tile (8 dims of one key).
 //   V slot: lane L takes head 2s + (L >> 5) and HD/64 consecutive 16-byte tile chunks: dims d and
 //   d + 16 of the four keys, loaded from the four rows and written with one store per chunk.
+//   q8_0: a K block of 32 values is a row's 8 lanes (amax over them, a word of codes per lane); a V
+//   block 16 / NF lanes, the four tokens' codes of a dim one word. f32: whole float4s.
+// Bound by HBM and, in short calls, by the chain of dependent reads (the staged row record first, which
+// holds the position and block id). 2,000 rows, 32/8 heads of 128, kernel us, row by row before / so:
+// q8_0 31.7 / 23.4, f32 29.0 / 24.1 (bf16: 23.0); 40 rows: 8.6 -> 7.2 (bf16 9.5 -> 7.1, records alone).
 // Slots y*spw .. y*spw+spw-1 of [Q pairs][K pairs][V pairs] are the workgroup's share.
-template <int HD, bool BF>
-__device__ void rope_quad_slots(const PageGeom& g, const RopeGeom& r, float2 (*cs)[ROPE_MAX_DIM / 2], uint32_t row0,
-                                uint32_t s0, uint32_t s1, const int32_t* row_seq, const int32_t* row_pos,
-                                const float* q, const float* k, const float* v, float* q_out) {
+template <int HD, int T>
+__device__ void rope_quad_slots(const PageGeom& g, const RopeGeom& r, float2 (*cs)[ROPE_MAX_DIM / 2], const RopeRow& rr,
+                                uint32_t s0, uint32_t s1, const float* q, const float* k, const float* v, float* q_out) {
   constexpr uint32_t NF = HD / 64, H2 = HD / 2;
   typedef float fc __attribute__((ext_vector_type(NF)));
   const uint32_t tid = threadIdx.x, lane = tid & 63u;
   const uint32_t w = __builtin_amdgcn_readfirstlane(tid >> 6);
   const uint32_t qs = (r.n_head + 1) / 2, ks = (g.n_kv + 1) / 2;
   const uint32_t sub = lane & 7u, hsel = (lane >> 3) & 1u, t = lane >> 4;
+  const uint32_t row0 = rr.row;
   const size_t row = row0 + t;
   const uint32_t q0 = (lane & 31u) * NF, d0 = 32u * (q0 >> 4) + (q0 & 15u);  // a V slot's dims
   // the values of slot sn, requested one slot ahead of their use (the first before the
@@ -799,7 +836,7 @@ __device__ void rope_quad_slots(const PageGeom& g, const RopeGeom& r, float2 (*c
   };
   float4 xn[2][NF];
   if (s0 + w < s1) load_slot(s0 + w, xn);
-  const uint32_t pos0 = (uint32_t)row_pos[row0];
+  const uint32_t pos0 = rr.pos;
   const uint32_t half = r.half_rot;
   for (uint32_t i = tid; i < 4 * half; i += blockDim.x) {
     const uint32_t tk = i / half, ii = i - tk * half;
@@ -809,7 +846,7 @@ __device__ void rope_quad_slots(const PageGeom& g, const RopeGeom& r, float2 (*c
     sincosf(angle, &sn, &cn);
     cs[tk][ii] = make_float2(cn * r.attn_factor, sn * r.attn_factor);
   }
-  const Slot sl0 = locate(g, row_seq[row0], pos0);
+  const Slot sl0 = locate(g, rr);
   __syncthreads();
   const bool neox = (r.flags & ROPE_NEOX) != 0;
   // rotation factors of the lane's elements, the same for every Q / K slot: Neox, element c of
@@ -894,8 +931,8 @@ __device__ void rope_quad_slots(const PageGeom& g, const RopeGeom& r, float2 (*c
           }
         }
       }
-      if (!on) continue;
       if (kind == 0) {
+        if (!on) continue;
         float* dst = q_out + (row * r.n_head + hh) * HD;
 #pragma unroll
         for (uint32_t hb = 0; hb < 2; hb++)
@@ -908,13 +945,27 @@ __device__ void rope_quad_slots(const PageGeom& g, const RopeGeom& r, float2 (*c
             __builtin_nontemporal_store(v, (f4*)(dst + hb * H2 + 4 * (sub + 8 * f)));
           }
       } else {
-        uint8_t* head = sl0.base + g.k_off + hh * g.k_head + sl0.tile * g.k_tile;
+        if (!on) continue;   // a row's 8 lanes alike
+        uint8_t* base = sl0.base + g.k_off + hh * g.k_head;
+        uint8_t* head = base + sl0.tile * g.k_tile;
 #pragma unroll
         for (uint32_t hb = 0; hb < 2; hb++)
 #pragma unroll
-          for (uint32_t f = 0; f < NF; f++)
-            *(uint2*)(head + k16_off(sl0.m + t, hb * H2 + 4 * (sub + 8 * f))) =
-                make_uint2(pack16x2<BF>(x[hb][f].x, x[hb][f].y), pack16x2<BF>(x[hb][f].z, x[hb][f].w));
+          for (uint32_t f = 0; f < NF; f++) {
+            const uint32_t d = hb * H2 + 4 * (sub + 8 * f);
+            if constexpr (T == KV_F32) {
+              *(float4*)(head + ((sl0.m + t) * HD + d) * 4) = x[hb][f];
+            } else if constexpr (T == KV_Q8) {   // a block of 32 values: the row's 8 lanes (quantize_q8_0, kv.rs:156-171)
+              const float amax = lanes8_max(fmaxf(fmaxf(fabsf(x[hb][f].x), fabsf(x[hb][f].y)), fmaxf(fabsf(x[hb][f].z), fabsf(x[hb][f].w))));
+              const float dsc = amax / 127.0f, id = dsc != 0.0f ? 1.0f / dsc : 0.0f;
+              *(uint32_t*)(head + kq8_off(sl0.m + t, d)) = q8x4(x[hb][f].x, x[hb][f].y, x[hb][f].z, x[hb][f].w, id);
+              if (sub == 0)
+                *(uint16_t*)(base + g.k_scale + sl0.tile * g.k_tile_s + ((sl0.m + t) * (HD / 32) + (d >> 5)) * 2u) = f16_bits(dsc);
+            } else {
+              *(uint2*)(head + k16_off(sl0.m + t, d)) =
+                  make_uint2(pack16x2<T == KV_BF16>(x[hb][f].x, x[hb][f].y), pack16x2<T == KV_BF16>(x[hb][f].z, x[hb][f].w));
+            }
+          }
       }
     } else {
       const uint32_t hv = 2 * (s - qs - ks) + (lane >> 5);
@@ -940,36 +991,69 @@ __device__ void rope_quad_slots(const PageGeom& g, const RopeGeom& r, float2 (*c
           }
         }
       }
-      if (!on) continue;
-      uint8_t* head = sl0.base + g.v_off + hv * g.v_head + sl0.tile * g.v_tile;
+      uint8_t* base = sl0.base + g.v_off + hv * g.v_head;
+      uint8_t* head = base + sl0.tile * g.v_tile;
+      if constexpr (T == KV_Q8) {
+        // a token's block of 32 values: 16 / NF lanes, each with dims d0 .. and d0 + 16 ..; a dim's codes
+        // of the four tokens are one word of the tile, d + 16's the next
+        uint32_t ca[NF], cb[NF];
 #pragma unroll
-      for (uint32_t c = 0; c < NF; c++)
-        *(uint4*)(head + v16_off(sl0.m, d0 + c)) =
-            make_uint4(pack16x2<BF>(a[0][c], a[1][c]), pack16x2<BF>(a[2][c], a[3][c]),
-                       pack16x2<BF>(b[0][c], b[1][c]), pack16x2<BF>(b[2][c], b[3][c]));
+        for (uint32_t c = 0; c < NF; c++) ca[c] = cb[c] = 0;
+#pragma unroll
+        for (uint32_t tt = 0; tt < 4; tt++) {
+          float amax = 0.f;
+#pragma unroll
+          for (uint32_t c = 0; c < NF; c++) amax = fmaxf(amax, fmaxf(fabsf(a[tt][c]), fabsf(b[tt][c])));
+          amax = lanes_max<16 / NF>(amax);
+          const float dsc = amax / 127.0f, id = dsc != 0.0f ? 1.0f / dsc : 0.0f;
+#pragma unroll
+          for (uint32_t c = 0; c < NF; c++) {
+            ca[c] |= (uint32_t)(uint8_t)(int8_t)(int32_t)rintf(a[tt][c] * id) << (8 * tt);
+            cb[c] |= (uint32_t)(uint8_t)(int8_t)(int32_t)rintf(b[tt][c] * id) << (8 * tt);
+          }
+          if (on && (q0 & 15u) == 0)
+            *(uint16_t*)(base + g.v_scale + sl0.tile * g.v_tile_s + ((sl0.m + tt) * (HD / 32) + (d0 >> 5)) * 2u) = f16_bits(dsc);
+        }
+        if (!on) continue;
+#pragma unroll
+        for (uint32_t c = 0; c < NF; c++) *(uint2*)(head + vq8_off(sl0.m, d0 + c)) = make_uint2(ca[c], cb[c]);
+        continue;
+      }
+      if (!on) continue;
+      if constexpr (T == KV_F32) {
+#pragma unroll
+        for (uint32_t tt = 0; tt < 4; tt++) {
+          *(fc*)(head + ((sl0.m + tt) * HD + d0) * 4) = a[tt];
+          *(fc*)(head + ((sl0.m + tt) * HD + d0 + 16) * 4) = b[tt];
+        }
+      } else {
+#pragma unroll
+        for (uint32_t c = 0; c < NF; c++)
+          *(uint4*)(head + v16_off(sl0.m, d0 + c)) =
+              make_uint4(pack16x2<T == KV_BF16>(a[0][c], a[1][c]), pack16x2<T == KV_BF16>(a[2][c], a[3][c]),
+                         pack16x2<T == KV_BF16>(b[0][c], b[1][c]), pack16x2<T == KV_BF16>(b[2][c], b[3][c]));
+      }
     }
   }
 }
 
 // The launch of rope_quad_slots: workgroups x < n_quads take an aligned run of 4 tokens and
 // slots y*spw .. ; the others one remaining row and items y*ipw .. (rope_tokens<HD / 64, 1>).
-template <int HD, bool BF>
-__global__ __launch_bounds__(256) void qk_rope_store_slots_kernel(PageGeom g, RopeGeom r, const int32_t* quads,
-                                                                  uint32_t n_quads, const int32_t* rest,
-                                                                  const int32_t* row_seq, const int32_t* row_pos,
-                                                                  const float* q, const float* k, const float* v,
-                                                                  float* q_out, uint32_t ipw, uint32_t spw) {
+template <int HD, int T>
+__global__ __launch_bounds__(256) void qk_rope_store_slots_kernel(PageGeom g, RopeGeom r, const RopeRow* quads,
+                                                                  uint32_t n_quads, const RopeRow* rest, const float* q,
+                                                                  const float* k, const float* v, float* q_out,
+                                                                  uint32_t ipw, uint32_t spw) {
   __shared__ float2 cs[4][ROPE_MAX_DIM / 2];
   if (blockIdx.x < n_quads) {
     const uint32_t n_slots = (r.n_head + 1) / 2 + 2 * ((g.n_kv + 1) / 2);
     const uint32_t s0 = blockIdx.y * spw, s1 = min(n_slots, s0 + spw);
     if (s0 >= s1) return;
-    rope_quad_slots<HD, BF>(g, r, cs, (uint32_t)quads[blockIdx.x], s0, s1, row_seq, row_pos, q, k, v, q_out);
+    rope_quad_slots<HD, T>(g, r, cs, quads[blockIdx.x], s0, s1, q, k, v, q_out);
   } else {
     const uint32_t it0 = blockIdx.y * ipw, n_items = min(r.n_head + 2 * g.n_kv, it0 + ipw);
     if (it0 >= n_items) return;
-    rope_tokens<HD / 64, 1>(g, r, cs, rest ? (uint32_t)rest[blockIdx.x - n_quads] : blockIdx.x - n_quads, it0,
-                            n_items, row_seq, row_pos, q, k, v, q_out);
+    rope_tokens<HD / 64, 1>(g, r, cs, rest[blockIdx.x - n_quads], it0, n_items, q, k, v, q_out);
   }
 }
 
@@ -1351,9 +1435,16 @@ hipError_t launch_gather_encoded(const PageGeom& g, const int32_t* row_seq, cons
   return hipGetLastError();
 }
 
+// Runs are taken whole from this many rows on: at once but for 256-wide heads on q8_0 and f32 pages,
+// where a short call is faster row by row (kernel us, runs / rows: f32 256 at 40 rows 9.0 / 7.8, at 200
+// 9.4 / 12.6; q8_0 128 at 40 7.2 / 7.5, at 400 8.8 / 14.5; bf16 128 at 4 6.1 / 7.5, at 400 9.2 / 13.6).
+inline uint32_t rope_run_rows(uint32_t kv_type, uint32_t hd) {
+  return hd == 256 && (kv_type == KV_Q8 || kv_type == KV_F32) ? 128 : 1;
+}
+
 hipError_t launch_qk_rope_store(const PageGeom& g, const RopeGeom& r, const int32_t* row_seq, const int32_t* row_pos,
                                 uint32_t n_rows, const float* q, const float* k, const float* v, float* q_out,
-                                const int32_t* quads, uint32_t n_quads, const int32_t* rest, uint32_t n_rest,
+                                const RopeRow* quads, uint32_t n_quads, const RopeRow* rest, uint32_t n_rest,
                                 hipStream_t s, const LaunchEv& ev) {
   if (n_rows == 0) return hipSuccess;
   // register path: hd == hdv = 64*VPL; Normal pairs are always in-lane (VPL >= 2) or one lane
@@ -1365,22 +1456,15 @@ hipError_t launch_qk_rope_store(const PageGeom& g, const RopeGeom& r, const int3
   const bool reg = g.layout == LAYOUT_TILES && g.hd == g.hdv && g.hd % 64 == 0 &&
                    (vpl == 1 || vpl == 2 || vpl == 4) && pairs_ok;
   if (reg) {
-    // aligned runs of 4 f16 / bf16 rows (when the caller found any) with the other rows, or a
-    // short call of any type (decode rows), go to the split kernel: one launch, each row's heads
-    // split over workgroups (8 items = one round of 2 heads per wave at the least) until the grid
-    // holds about 1024 workgroups, the 4 per CU its registers allow (measured on 256 .. 8192 rows:
-    // a target of 512 or 2048 is slower at 2048 and 4096 rows). Long calls without runs go to the
-    // row kernel, which keeps 16 heads per wave in flight.
-    const bool quad_ok = n_quads > 0 && (g.kv_type == KV_F16 || g.kv_type == KV_BF16);
-    if (!quad_ok) {
-      n_quads = 0;
-      rest = nullptr;
-      n_rest = n_rows;
-    }
+    // aligned runs of 4 rows (when the caller found any) with the other rows, or a short call's rows one
+    // by one, go to the split kernels: one launch, each row's heads split over workgroups (8 items = one
+    // round of 2 heads per wave at the least) until the grid holds about 1024 workgroups, the 4 per CU
+    // its registers allow (measured on 256 .. 8192 rows: a target of 512 or 2048 is slower at 2048 and
+    // 4096 rows). Long calls without runs go to the row kernel, which keeps 16 heads per wave in flight.
     // the slot kernel: hd == hdv in {64, 128, 256}, rotated pairs inside a lane (Normal, or Neox
     // over all dims), every row and weight vector 16-byte aligned
     const auto al16 = [](const void* p) { return ((uintptr_t)p & 15u) == 0; };
-    const bool slots = quad_ok && g.hd == g.hdv && (g.hd == 64 || g.hd == 128 || g.hd == 256) &&
+    const bool slots = n_quads > 0 && n_rows >= rope_run_rows(g.kv_type, g.hd) && g.hd == g.hdv && (g.hd == 64 || g.hd == 128 || g.hd == 256) &&
                        (!neox || half == 0 || half == g.hd / 2) && r.q_stride % 4 == 0 && al16(q) && al16(k) &&
                        al16(v) && al16(q_out) && al16(r.q_norm) && al16(r.k_norm);
     if (slots) {
@@ -1392,25 +1476,35 @@ hipError_t launch_qk_rope_store(const PageGeom& g, const RopeGeom& r, const int3
       const uint32_t split = std::min(max_split, std::max(1u, (1024u + n_wg - 1) / n_wg));
       const uint32_t spw = (n_slots + split - 1) / split, ipw = ((n_items + split - 1) / split + 3) & ~3u;
       const dim3 grid(n_wg, std::max((n_slots + spw - 1) / spw, (n_items + ipw - 1) / ipw));
-#define LMH_SLOTS(H, B)                                                                                            \
-  LMH_LAUNCH(ev, (qk_rope_store_slots_kernel<H, B>), grid, dim3(256), 0, s, g, r, quads, n_quads, rest, row_seq, \
-             row_pos, q, k, v, q_out, ipw, spw)
-      const bool bf = g.kv_type == KV_BF16;
+#define LMH_SLOTS(H, T)                                                                                            \
+  LMH_LAUNCH(ev, (qk_rope_store_slots_kernel<H, T>), grid, dim3(256), 0, s, g, r, quads, n_quads, rest, q, k, v, \
+             q_out, ipw, spw)
+#define LMH_SLOTS_T(H)                     \
+  switch (g.kv_type) {                     \
+    case KV_F16: LMH_SLOTS(H, KV_F16); break;   \
+    case KV_BF16: LMH_SLOTS(H, KV_BF16); break; \
+    case KV_Q8: LMH_SLOTS(H, KV_Q8); break;     \
+    default: LMH_SLOTS(H, KV_F32); break;       \
+  }
       switch (g.hd) {
-        case 64: if (bf) LMH_SLOTS(64, true); else LMH_SLOTS(64, false); break;
-        case 128: if (bf) LMH_SLOTS(128, true); else LMH_SLOTS(128, false); break;
-        default: if (bf) LMH_SLOTS(256, true); else LMH_SLOTS(256, false); break;
+        case 64: LMH_SLOTS_T(64); break;
+        case 128: LMH_SLOTS_T(128); break;
+        default: LMH_SLOTS_T(256); break;
       }
+#undef LMH_SLOTS_T
 #undef LMH_SLOTS
       return hipGetLastError();
     }
-    if (quad_ok || n_rows < 1024) {
-      const uint32_t n_wg = n_quads + n_rest, n_items = r.n_head + 2 * g.n_kv, max_split = (n_items + 7) / 8;
+    // runs whole on 16-bit pages (8-byte V words), else taken apart
+    const bool runs = n_quads > 0 && (g.kv_type == KV_F16 || g.kv_type == KV_BF16);
+    if (runs || n_rows < 1024) {
+      const uint32_t n_apart = runs ? 0 : n_quads, n_wg = (runs ? n_quads : 4 * n_quads) + n_rest;
+      const uint32_t n_items = r.n_head + 2 * g.n_kv, max_split = (n_items + 7) / 8;
       const uint32_t split = std::min(max_split, std::max(1u, (1024u + n_wg - 1) / n_wg));
       const uint32_t ipw = ((n_items + split - 1) / split + 3) & ~3u;
       const dim3 grid(n_wg, (n_items + ipw - 1) / ipw);
-#define LMH_QUAD(V)                                                                                            \
-  LMH_LAUNCH(ev, qk_rope_store_quad_kernel<V>, grid, dim3(256), 0, s, g, r, quads, n_quads, rest, row_seq, row_pos, \
+#define LMH_QUAD(V)                                                                                             \
+  LMH_LAUNCH(ev, qk_rope_store_quad_kernel<V>, grid, dim3(256), 0, s, g, r, quads, runs ? n_quads : 0u, n_apart, rest, \
              q, k, v, q_out, ipw)
       switch (vpl) {
         case 1: LMH_QUAD(1); break;
