@@ -742,6 +742,13 @@ extern "C" {
 
 const char* lmh_create_error(void) { return g_create_error.c_str(); }
 
+// Bytes a staging slot holds from the start, and what n_rows' (sequence, position) arrays leave of them.
+static size_t staging_bytes(uint64_t bps) { return std::max<size_t>(1 << 20, bps * 4 * 16); }
+static uint64_t list_bytes(size_t slot, uint64_t n_rows) {
+  const size_t rows = (n_rows * 8 + 255) / 256 * 256;
+  return slot - std::min(slot, rows);
+}
+
 int32_t lmh_kv_create(const lmh_kv_options* o, lmh_kv** out) {
   g_create_error.clear();
   if (!o || !out) {
@@ -874,7 +881,7 @@ int32_t lmh_kv_create(const lmh_kv_options* o, lmh_kv** out) {
   if (e == hipSuccess && kv->window) e = hipMalloc((void**)&kv->d_wtable, kv->h_wtable.size() * 4);
   // staging slots sized for a call's work list (decode items, merges, prefill units: 1 MiB holds
   // ~32 K decode items) and 16 block-table rows, so calls do not grow them
-  if (e == hipSuccess) e = kv->up.reserve(std::max<size_t>(1 << 20, kv->bps * 4 * 16));
+  if (e == hipSuccess) e = kv->up.reserve(staging_bytes(kv->bps));
   // this device's copy of lmh_attend_noalloc's scratch (resolved once per device)
   if (e == hipSuccess) e = noalloc_scratch(o->device, &kv->scratch);
   if (e == hipSuccess) {
@@ -1474,6 +1481,7 @@ static int32_t attend_impl(lmh_kv* kv, uint32_t layer, const lmh_seg* segs, uint
   pin.prefill_no_split = kv->prefill_whole_units;
   pin.noalloc = noalloc;
   pin.noalloc_bytes = NOALLOC_SCRATCH_BYTES;
+  pin.noalloc_stage = list_bytes(kv->up.reserved, n_rows);
   fill_kernel_facts(pin, kv->kv_type, y.hd, y.hdv, group, y.layout);
   for (uint32_t nb = 1; nb <= 2; nb++) {
     if (!pin.unit_w[nb - 1]) continue;
@@ -1484,7 +1492,6 @@ static int32_t attend_impl(lmh_kv* kv, uint32_t layer, const lmh_seg* segs, uint
   PlanOut& pl = kv->plan;
   plan_attend(pin, pl);
   const uint32_t ng = pl.ng, slots = pl.slots, pf_wg = pl.pf_wg, pf_per_wg = pl.pf_per_wg, max_pages = pl.max_pages;
-  const bool local = pl.local != 0;
   const size_t slot_bytes = (size_t)ng * (y.hdv + 4) * 4;
   if ((rc = kv->flush(st)) != LMH_OK) return rc;
   const size_t items_bytes = kv->plan.items.size() * sizeof(DecodeItem);
@@ -1710,6 +1717,7 @@ int32_t lmh_plan_attend(const lmh_plan_desc* d, const lmh_seg* segs, uint64_t n_
   in.prefill_no_split = d->tuning.prefill_whole_units != 0;
   in.noalloc = d->noalloc != 0;
   in.noalloc_bytes = NOALLOC_SCRATCH_BYTES;
+  in.noalloc_stage = list_bytes(staging_bytes(in.bps), n_rows);
   in.list_units = true;
   fill_kernel_facts(in, d->kv_type, d->hd, d->hdv, d->n_head / d->n_kv, in.layout);
   PlanOut o;

@@ -297,6 +297,12 @@ bool plan_units(const PlanIn& in, PlanOut& o) {
   // Workgroup b runs on XCD b % 8: in one round, runs of consecutive workgroups go to one XCD, so
   // units that read the same pages (a KV head's are consecutive) share its L2.
   const uint32_t n_xcd = in.n_cu % 8 == 0 && !rounds ? 8 : 1, per_xcd = (n_wg + n_xcd - 1) / n_xcd;
+  // A wave's record is longer than a decode item's: calls of many single rows whose list of items fits
+  // the staging of an allocation-free call, and this one not, stay on the decode items.
+  if (in.noalloc && (uint64_t)per_xcd * n_xcd * W * sizeof(UnitWave) > in.noalloc_stage) {
+    o.u_nb = o.u_w = 0;
+    return false;
+  }
   auto launch_at = [&](uint32_t wg) { return n_xcd == 1 ? wg : wg % per_xcd * n_xcd + wg / per_xcd; };
   // partial slots and merges of the units in several pieces (their members are consecutive), the heads
   // of a merge few enough for about a thousand merge waves

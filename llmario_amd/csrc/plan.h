@@ -50,6 +50,7 @@ struct PlanIn {
   bool mfma_local_ok = false;       // matrix-core decode: the same, for rows split at most 4 ways
   uint32_t unit_w[2] = {0, 0};      // most waves per workgroup of the unit launch of 16 / 32 columns (0: no instance)
   uint32_t unit_waves_per_cu[2] = {8, 8};   // its waves a CU holds at once
+  uint64_t noalloc_stage = ~0ull;   // noalloc: bytes of work list that fit the staging reserved at creation
   bool list_units = false;          // list the unit launch's units in pitems too (lmh_plan_attend)
 };
 

@@ -75,3 +75,17 @@ def test_long_units_are_cut_and_short_ones_packed():
     items, merges, units, c = plan("f16", 32, 8, 128, 128, 16, table, segs)
     check_plan("f16", 32, 8, 128, 128, 16, table, segs, 0, items, merges, units, c)
     assert c.slots == 0 and len(merges) == 0 and len(items) == 0 and c.pf_wg <= 512
+
+
+def test_allocation_free_calls_keep_a_list_that_fits():
+    """The staging an allocation-free call may use (1 MiB here) takes 900 single rows of 32 KV heads as
+    decode items, not as unit records; fewer rows, and calls that may allocate, are units."""
+    geo = (32, 32, 80, 80)
+    for n, noalloc, units_expected in ((900, True, False), (900, False, True), (500, True, True)):
+        table = contiguous_table([21] * n, 16)
+        segs = [(i, i, 1, 20) for i in range(n)]
+        items, merges, units, c = plan("f16", *geo, 16, table, segs, noalloc=noalloc)
+        assert (len(units) > 0) == units_expected and (len(items) > 0) != units_expected, (n, noalloc)
+        if len(items):
+            assert len(items) * 32 + n * 8 <= 1 << 20
+        check_plan("f16", *geo, 16, table, segs, 0, items, merges, units, c, noalloc=noalloc)
