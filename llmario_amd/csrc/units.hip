@@ -23,7 +23,7 @@
 // Measured, one step of lmh_attend, against a decode item per row (before; the row layout's and f32
 // pages' on the VALU): 24 sequences x 4 rows on 512 .. 4,096 keys (32/8 heads, hd 128, bf16, 190 MB of
 // pages): 98.5 -> 41.5 us (5.9 TB/s at four times the contexts: bound by HBM, the rest start-up and the
-// cut units' merge); hd 256 prompts of 600 and 800 tokens, window 1,024: 225 -> 57 us, two of 2,048:
+// cut units' merge); hd 256 prompts of 600 and 800 tokens, window 1,024: 225 -> 63 us (57 before non-finite V of a masked key was kept out), two of 2,048:
 // 410 TFLOP/s (bound by the matrix cores and one wave's latency per SIMD); hd 80, 32 heads of their own
 // K/V, 8 decode rows and a 120-token chunk: 1,038 -> 30 us (decode rows alone at 8,000 keys: 5.0 TB/s);
 // f32 prompts of 450 and 390 tokens, hd 64: 102 -> 23 us. The row layout's loads are ordinary ones:
@@ -455,28 +455,34 @@ __device__ __forceinline__ void unit_wave(const PageGeom& g, const UnitGeom& u, 
           for (int kk = 0; kk < KT; kk++)
             lsum[x] += (p[x][4 * kk] + p[x][4 * kk + 1]) + (p[x][4 * kk + 2] + p[x][4 * kk + 3]);
         }
-        // Row layout and f32 pages: a key some columns do not see may hold anything (a later row's
-        // value, or what an earlier owner of the page left), and 0 * inf is not 0. Non-finite values of
-        // such a step stay out of its products, and reach the columns that see them afterwards.
+        // A key some columns do not see may hold anything (a later row's value, or what an earlier owner
+        // of the page left), and 0 * inf is not 0. Non-finite values of such a step stay out of its
+        // products, and reach the columns that see them afterwards. (bf16 tiles: values beyond f16's
+        // range too, as their products are taken in f16. q8_0 values are finite below 8e6.)
         bool bad_v = false;
         auto nonfinite = [](uint32_t v) -> uint32_t {   // mask of the word's non-finite values
           if constexpr (F32) return (v & 0x7f800000u) == 0x7f800000u ? ~0u : 0u;
-          constexpr uint32_t E = BF ? 0x7f80u : 0x7c00u;
-          return ((v & E) == E ? 0xffffu : 0u) | (((v >> 16) & E) == E ? 0xffff0000u : 0u);
+          constexpr uint32_t E = F == FT_BF16 ? 0x4780u : BF ? 0x7f80u : 0x7c00u;   // the least non-finite magnitude
+          return ((v & 0x7fffu) >= E ? 0xffffu : 0u) | ((v & 0x7fff0000u) >= E << 16 ? 0xffff0000u : 0u);
         };
-        if constexpr (ROWS) {
+        if constexpr (!Q8) {
           if (need_mask) {
-            uint32_t any = 0;
+            // the largest magnitude (two operations a word: the step waits for it)
+            typedef uint16_t u16x2 __attribute__((ext_vector_type(2)));
+            typename std::conditional<F32, uint32_t, u16x2>::type top = 0;
 #pragma unroll
             for (int b = 0; b < C::VR; b++) {
 #pragma unroll
               for (int kk = 0; kk < KT; kk++) {
                 const uint32_t* v = (const uint32_t*)&vr[kk][b];
 #pragma unroll
-                for (int i = 0; i < 4; i++) any |= nonfinite(v[i]);
+                for (int i = 0; i < 4; i++) {
+                  if constexpr (F32) top = max(top, v[i] & 0x7fffffffu);
+                  else top = __builtin_elementwise_max(top, __builtin_bit_cast(u16x2, v[i] & 0x7fff7fffu));
+                }
               }
             }
-            bad_v = __ballot(any != 0) != 0;
+            bad_v = __ballot(nonfinite(__builtin_bit_cast(uint32_t, top)) != 0) != 0;
             if (bad_v) {
 #pragma unroll
               for (int b = 0; b < C::VR; b++) {
@@ -606,73 +612,76 @@ __device__ __forceinline__ void unit_wave(const PageGeom& g, const UnitGeom& u, 
             }
           }
         }
-        if constexpr (ROWS) {
+        if constexpr (!Q8) {
           if (bad_v) {
             // how many NaN, +inf and -inf values of a dim a column sees: products of 0 / 1 operands
             ids(st);
             bases(st);
 #pragma unroll
             for (int b = 0; b < C::VR; b++) load_v(b);
-            float see[NB][4 * KT];
+            float see[NB][F32 ? 4 : 1];
+            h8 seeh[NB];
 #pragma unroll
             for (int x = 0; x < NB; x++)
 #pragma unroll
-              for (int kk = 0; kk < KT; kk++)
-#pragma unroll
-                for (int r = 0; r < 4; r++) {
-                  const uint32_t key = key0 + 16 * kk + 4 * grp + r;
-                  see[x][4 * kk + r] = key <= cpos[x] && key >= clo[x] && key < page_end << 4 ? 1.0f : 0.0f;
-                }
-            auto kind = [](float v, int k) -> float {   // k: 0 NaN, 1 +inf, 2 -inf
-              return (k == 0 ? v != v : v == (k == 1 ? INFINITY : -INFINITY)) ? 1.0f : 0.0f;
+              for (int i = 0; i < 4 * KT; i++) {
+                const uint32_t key = key0 + 16 * (i >> 2) + 4 * grp + (i & 3);
+                const bool on = key <= cpos[x] && key >= clo[x] && key < page_end << 4;
+                if constexpr (F32) see[x][i] = on ? 1.0f : 0.0f;
+                else seeh[x][i] = on ? (_Float16)1.0f : (_Float16)0.0f;
+              }
+            auto kind = [](float v, int k) -> float {   // k: 0 +inf, 1 -inf, 2 NaN
+              constexpr float TOP = F == FT_BF16 ? 65536.f : INFINITY;
+              return (k == 2 ? v != v : k == 0 ? v >= TOP : v <= -TOP) ? 1.0f : 0.0f;
             };
 #pragma unroll
             for (int j = 0; j < NJ; j++) {
               __builtin_amdgcn_sched_barrier(0);   // one block at a time: no registers to spare
-              f4 cnt[3][NB];
 #pragma unroll
               for (int k = 0; k < 3; k++) {
+                f4 cnt[NB];
 #pragma unroll
-                for (int x = 0; x < NB; x++) cnt[k][x] = f4{0.f, 0.f, 0.f, 0.f};
+                for (int x = 0; x < NB; x++) cnt[x] = f4{0.f, 0.f, 0.f, 0.f};
                 if constexpr (F32) {
 #pragma unroll
                   for (int r = 0; r < 4; r++) {
                     const f4 v = __builtin_bit_cast(f4, vr[0][4 * (j / 4) + r]);
 #pragma unroll
                     for (int x = 0; x < NB; x++)
-                      cnt[k][x] = __builtin_amdgcn_mfma_f32_16x16x4f32(kind(v[j & 3], k), see[x][r], cnt[k][x], 0, 0, 0);
+                      cnt[x] = __builtin_amdgcn_mfma_f32_16x16x4f32(kind(v[j & 3], k), see[x][r], cnt[x], 0, 0, 0);
                   }
                 } else {
                   h8 a;
 #pragma unroll
                   for (int i = 0; i < 8; i++) {
-                    const uint32_t w32 = ((const uint32_t*)&vr[i >> 2][j >> 1])[i & 3];
-                    const uint16_t w16 = (uint16_t)((j & 1) ? w32 >> 16 : w32);
+                    // rows: a word per key, its halves two blocks; tiles: a half per key
+                    const uint32_t* vw = (const uint32_t*)&vr[i >> 2][j >> 1];
+                    const uint32_t w32 = ROWS ? vw[i & 3] : vw[2 * (j & 1) + ((i & 3) >> 1)];
+                    const uint16_t w16 = (uint16_t)(((ROWS ? j : i) & 1) ? w32 >> 16 : w32);
                     a[i] = (_Float16)kind(BF ? __uint_as_float((uint32_t)w16 << 16) : h_to_f(w16), k);
                   }
 #pragma unroll
-                  for (int x = 0; x < NB; x++) {
-                    h8 sv;
-#pragma unroll
-                    for (int i = 0; i < 8; i++) sv[i] = (_Float16)see[x][i];
-                    cnt[k][x] = __builtin_amdgcn_mfma_f32_16x16x32_f16(a, sv, cnt[k][x], 0, 0, 0);
-                  }
+                  for (int x = 0; x < NB; x++) cnt[x] = __builtin_amdgcn_mfma_f32_16x16x32_f16(a, seeh[x], cnt[x], 0, 0, 0);
                 }
+                constexpr uint32_t ADD[3] = {0x7f800000u, 0xff800000u, 0x7fc00000u};
+#pragma unroll
+                for (int x = 0; x < NB; x++)
+#pragma unroll
+                  for (int r = 0; r < 4; r++) O[x][j][r] += cnt[x][r] > 0.f ? __uint_as_float(ADD[k]) : 0.f;
               }
-#pragma unroll
-              for (int x = 0; x < NB; x++)
-#pragma unroll
-                for (int r = 0; r < 4; r++) {
-                  const bool nan = cnt[0][x][r] > 0.f, pi = cnt[1][x][r] > 0.f, ni = cnt[2][x][r] > 0.f;
-                  if (nan || pi || ni) O[x][j][r] += nan || (pi && ni) ? __uint_as_float(0x7fc00000u) : pi ? INFINITY : -INFINITY;
-                }
             }
             ids(st + 1);
             bases(st + 1);
             ids(st + 2);
-          }
+            if constexpr (!ROWS && !F32) {
 #pragma unroll
-          for (int b = 0; b < C::VR; b++) load_v(b);
+              for (int b = 0; b < C::VR; b++) load_v(b);
+            }
+          }
+          if constexpr (ROWS) {
+#pragma unroll
+            for (int b = 0; b < C::VR; b++) load_v(b);
+          }
         }
       }
       if constexpr (!Q8) break;
@@ -848,18 +857,25 @@ uint32_t unit_waves(uint32_t kv_type, uint32_t hd, uint32_t hdv, uint32_t layout
   return w;
 }
 
+// Asked of the runtime once per kernel (a query takes ~10 us, which each new cache's first call paid).
 uint32_t unit_waves_per_cu(uint32_t kv_type, uint32_t hd, uint32_t hdv, uint32_t layout, uint32_t nb) {
-  int blocks = 0;
+  uint32_t n = 4;
   auto ask = [&](auto f, auto a, auto b, auto nbt) {   // without LDS, 4-wave workgroups: what the registers allow
     constexpr int F = decltype(f)::value, A = decltype(a)::value, B = decltype(b)::value, NB = decltype(nbt)::value;
-    if constexpr (NB == 1 || two_blocks<F, A, B>())
-      if (hipOccupancyMaxActiveBlocksPerMultiprocessor(&blocks, unit_kernel<F, A, B, NB>, 256, 0) != hipSuccess) blocks = 0;
+    if constexpr (NB == 1 || two_blocks<F, A, B>()) {
+      static const uint32_t waves = [] {
+        int blocks = 0;
+        if (hipOccupancyMaxActiveBlocksPerMultiprocessor(&blocks, unit_kernel<F, A, B, NB>, 256, 0) != hipSuccess) blocks = 0;
+        return 4 * (uint32_t)std::max(blocks, 1);
+      }();
+      n = waves;
+    }
   };
   with_instance(kv_type, hd, hdv, layout, [&](auto f, auto a, auto b) {
     if (nb == 1) ask(f, a, b, std::integral_constant<int, 1>{});
     else ask(f, a, b, std::integral_constant<int, 2>{});
   });
-  return 4 * (uint32_t)std::max(blocks, 1);
+  return n;
 }
 
 hipError_t launch_units(const PageGeom& g, const UnitGeom& u, uint32_t nb, uint32_t w, const UnitWave* waves, uint32_t n_wg,

@@ -121,3 +121,32 @@ def test_a_row_ignores_values_it_does_not_see(cuda, kv, geo, bad):
     sees = (pos >= at) & (pos < at + window)
     assert np.array_equal(got[~sees], base[~sees])
     assert not np.isfinite(got[sees]).any()
+
+
+# f16 / bf16 tiles: runs of drafted tokens across a tile's end, prompts at either edge of a window.
+# 1e5 is beyond f16, in which the tiles' products are taken.
+@pytest.mark.parametrize("kv,geo,prior,new,window,at", [
+    ("f16", (32, 8, 128, 128), 3005, 7, 0, 3009), ("bf16", (32, 8, 128, 128), 3005, 7, 0, 3009),
+    ("f16", (32, 32, 64, 64), 3005, 6, 0, 3010), ("bf16", (16, 4, 256, 256), 1000, 70, 1000, 1040),
+    ("f16", (16, 4, 256, 256), 1000, 70, 1000, 30), ("bf16", (12, 4, 96, 96), 1000, 90, 0, 1017)])
+@pytest.mark.parametrize("bad", [float("inf"), float("-inf"), float("nan"), 1e5])
+def test_a_row_on_tiles_ignores_values_it_does_not_see(cuda, kv, geo, prior, new, window, at, bad):
+    import torch
+
+    w = small("ut", kv, Layer(*geo), prior=[prior] * 4, new=[new] * 4, window=window, seed=91)
+    hc, oc, q = pair(w)
+    base, kt = launches(hc, lambda: run_gpu(hc, w, q))
+    assert kt["prefill"][1] == 1 and kt["decode"][1] == 0, kt
+    L = w.layer
+    k, v = (torch.empty((1, L.n_kv * d), device="cuda") for d in (L.hd, L.hdv))
+    hc.gather(0, [(1, 0, 1, at)], k, v)
+    v[:] = bad
+    hc.store(0, [(1, 0, 1, at)], k, v)
+    got = run_gpu(hc, w, q)
+    pos = prior + np.arange(4 * new) - new
+    sees = (np.arange(4 * new) // new == 1) & (pos >= at)
+    if window:
+        sees &= pos < at + window
+    assert 0 < sees.sum() < new
+    assert np.array_equal(got[~sees], base[~sees])
+    assert not np.isfinite(got[sees]).any()
