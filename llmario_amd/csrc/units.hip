@@ -23,7 +23,8 @@
 // Measured, one step of lmh_attend, against a decode item per row (before; the row layout's and f32
 // pages' on the VALU): 24 sequences x 4 rows on 512 .. 4,096 keys (32/8 heads, hd 128, bf16, 190 MB of
 // pages): 98.5 -> 41.5 us (5.9 TB/s at four times the contexts: bound by HBM, the rest start-up and the
-// cut units' merge); hd 256 prompts of 600 and 800 tokens, window 1,024: 225 -> 63 us (57 before non-finite V of a masked key was kept out), two of 2,048:
+// cut units' merge); hd 256 prompts of 600 and 800 tokens, window 1,024: 225 -> 62 us (57 before
+// non-finite V of a masked key was kept out: the masked steps wait for V to test it), two of 2,048:
 // 410 TFLOP/s (bound by the matrix cores and one wave's latency per SIMD); hd 80, 32 heads of their own
 // K/V, 8 decode rows and a 120-token chunk: 1,038 -> 30 us (decode rows alone at 8,000 keys: 5.0 TB/s);
 // f32 prompts of 450 and 390 tokens, hd 64: 102 -> 23 us. The row layout's loads are ordinary ones:
@@ -483,7 +484,7 @@ __device__ __forceinline__ void unit_wave(const PageGeom& g, const UnitGeom& u, 
               }
             }
             bad_v = __ballot(nonfinite(__builtin_bit_cast(uint32_t, top)) != 0) != 0;
-            if (bad_v) {
+            if (__builtin_expect(bad_v, 0)) {
 #pragma unroll
               for (int b = 0; b < C::VR; b++) {
 #pragma unroll
@@ -613,7 +614,7 @@ __device__ __forceinline__ void unit_wave(const PageGeom& g, const UnitGeom& u, 
           }
         }
         if constexpr (!Q8) {
-          if (bad_v) {
+          if (__builtin_expect(bad_v, 0)) {
             // how many NaN, +inf and -inf values of a dim a column sees: products of 0 / 1 operands
             ids(st);
             bases(st);
@@ -673,7 +674,9 @@ __device__ __forceinline__ void unit_wave(const PageGeom& g, const UnitGeom& u, 
             ids(st + 1);
             bases(st + 1);
             ids(st + 2);
-            if constexpr (!ROWS && !F32) {
+            if constexpr (!ROWS && !F32) {   // (K again too: its registers are free in between)
+#pragma unroll
+              for (int c = 0; c < C::KR; c++) load_k(c);
 #pragma unroll
               for (int b = 0; b < C::VR; b++) load_v(b);
             }
