@@ -118,9 +118,9 @@ bool plan_units(const PlanIn& in, PlanOut& o) {
   // 5 rows of 6,000 24.4 -> 20.3, saves 11; 32 x 3 of 700 43.2 -> 23.6, saves 22).
   if (in.layout == LAYOUT_TILES && !f32 && (steps_rows - std::min(steps_rows, in.unit_w[1] ? steps32 : steps16)) * in.n_kv < 40ull * in.n_cu)
     return false;
-  o.ng = (uint32_t)std::min<uint64_t>(group, 16);   // a partial slot holds the group's heads (pieces: group <= 16)
-  o.u_nb = in.unit_w[1] && 4 * steps32 < 3 * steps16 ? 2 : 1;
-  const uint32_t KT = f32 ? 1 : 2, cols = 16 * o.u_nb;
+  // (o is written once the call is taken: one given back keeps what the other planners set)
+  const uint32_t nb = in.unit_w[1] && 4 * steps32 < 3 * steps16 ? 2 : 1;
+  const uint32_t KT = f32 ? 1 : 2, cols = 16 * nb;
   // A segment's column blocks; a unit is a block for one KV head.
   struct Block {
     PrefillItem it;
@@ -157,9 +157,8 @@ bool plan_units(const PlanIn& in, PlanOut& o) {
   const uint64_t n_units = (uint64_t)blocks.size() * in.n_kv;
   // Workgroups of the most waves share the longest units; where most units have a wave of their own
   // anyway, smaller ones leave a CU's waves to finish and start independently.
-  const uint32_t w_max = in.unit_w[o.u_nb - 1], per_cu = std::max(in.unit_waves_per_cu[o.u_nb - 1], w_max);
+  const uint32_t w_max = in.unit_w[nb - 1], per_cu = std::max(in.unit_waves_per_cu[nb - 1], w_max);
   const uint32_t W = 2 * n_units > (uint64_t)in.n_cu * per_cu ? std::min(4u, w_max) : w_max;
-  o.u_w = W;
   const uint64_t wg_cap = (uint64_t)in.n_cu * (per_cu / W), target = wg_cap * W;
   // More units than the device holds waves (or nearly, of very uneven lengths): several rounds.
   // (hd 64 f32 prompts of 2,048 tokens, 2,048 units of 1 .. 128 steps: 207 us in rounds, 241 as one;
@@ -299,10 +298,10 @@ bool plan_units(const PlanIn& in, PlanOut& o) {
   const uint32_t n_xcd = in.n_cu % 8 == 0 && !rounds ? 8 : 1, per_xcd = (n_wg + n_xcd - 1) / n_xcd;
   // A wave's record is longer than a decode item's: calls of many single rows whose list of items fits
   // the staging of an allocation-free call, and this one not, stay on the decode items.
-  if (in.noalloc && (uint64_t)per_xcd * n_xcd * W * sizeof(UnitWave) > in.noalloc_stage) {
-    o.u_nb = o.u_w = 0;
-    return false;
-  }
+  if (in.noalloc && (uint64_t)per_xcd * n_xcd * W * sizeof(UnitWave) > in.noalloc_stage) return false;
+  o.ng = (uint32_t)std::min<uint64_t>(group, 16);   // a partial slot holds the group's heads (pieces: group <= 16)
+  o.u_nb = nb;
+  o.u_w = W;
   auto launch_at = [&](uint32_t wg) { return n_xcd == 1 ? wg : wg % per_xcd * n_xcd + wg / per_xcd; };
   // partial slots and merges of the units in several pieces (their members are consecutive), the heads
   // of a merge few enough for about a thousand merge waves

@@ -89,3 +89,14 @@ def test_allocation_free_calls_keep_a_list_that_fits():
         if len(items):
             assert len(items) * 32 + n * 8 <= 1 << 20
         check_plan("f16", *geo, 16, table, segs, 0, items, merges, units, c, noalloc=noalloc)
+
+
+def test_a_call_given_back_keeps_the_items_head_blocks():
+    """Too many single rows for the staging of an allocation-free call, in a group wider than the
+    row-layout kernel's 4 heads per item: its items hold 4 heads each."""
+    geo, n = (128, 16, 80, 80), 1700
+    table = contiguous_table([21] * n, 16)
+    segs = [(i, i, 1, 20) for i in range(n)]
+    items, merges, units, c = plan("f16", *geo, 16, table, segs, noalloc=True)
+    assert len(units) == 0 and len(items) == n * 16 * 2 and c.ng == 4
+    check_plan("f16", *geo, 16, table, segs, 0, items, merges, units, c, noalloc=True)
