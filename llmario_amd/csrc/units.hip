@@ -137,7 +137,7 @@ __device__ __forceinline__ void unit_wave(const PageGeom& g, const UnitGeom& u, 
     ct[x] = cv[x] ? (c + c_off) / G : 0;
     ch[x] = cv[x] ? (c + c_off) - ct[x] * G : 0;
   }
-  float m[NB], lsum[NB], pup = 7.0f;
+  float m[NB], lsum[NB], pup[NB];
   f4 O[NB][NJ];
   if (n_share != 0) {
     const uint32_t pos0 = fld(2), page0 = fld(3), n_pages = fld(4);
@@ -310,12 +310,16 @@ __device__ __forceinline__ void unit_wave(const PageGeom& g, const UnitGeom& u, 
     }
 
     // pup, `checked`: as decode_item's (q8_0: weight x V scale in f16 range; a product that
-    // overflowed leaves O non-finite and the unit runs again with every step's scales checked)
+    // overflowed leaves O non-finite and the unit runs again with every step's scales checked), but of a
+    // column's own keys: the largest scale of the first step in which it sees one.
     bool checked = false;
+    uint32_t bad_blk[NB];   // q8_0: the 32-dim blocks for which a column sees a key of a non-finite V scale
     for (;;) {
-      pup = Q8 ? INFINITY : 7.0f;
+      bool unset = true;    // q8_0, uniform: some column has seen no key yet
 #pragma unroll
       for (int x = 0; x < NB; x++) {
+        pup[x] = Q8 ? INFINITY : 7.0f;
+        bad_blk[x] = 0;
         m[x] = -INFINITY;
         lsum[x] = 0.f;
 #pragma unroll
@@ -423,33 +427,100 @@ __device__ __forceinline__ void unit_wave(const PageGeom& g, const UnitGeom& u, 
             m[x] = mn;
           }
         }
+        // whether column x sees the lane's key i (of page tile i / 4). k0: the lane's first key, from
+        // lane_key(), which hides it: a test here is made again, rather than kept since the masks above.
+        auto lane_key = [&] {
+          uint32_t k0 = key0 + 4 * grp;
+          asm volatile("" : "+v"(k0));
+          return k0;
+        };
+        auto sees = [&](int x, int i, uint32_t k0) -> bool {
+          const uint32_t key = k0 + 16 * (i >> 2) + (i & 3);
+          return key <= cpos[x] && key >= clo[x] && key < page_end << 4;
+        };
         if constexpr (Q8) {
-          if (checked || st == 0) {   // uniform: the first step, or every step after an overflow
-            uint32_t mx = 0;
+          // A scale that is not finite (a value beyond 8.3e6) would make NaN of a weight of 0: on the steps
+          // where a column does not see every key, such scales stay out of the products, and the columns
+          // that see the key get their NaN at the end.
+          auto half_at = [&](int i, int b) -> uint32_t {
+            const int at = (i & 3) * NCH + b;
+            const uint32_t wv = ((const uint32_t*)vs[i >> 2])[at >> 1];
+            return ((at & 1) ? wv >> 16 : wv) & 0x7fffu;
+          };
+          if (need_mask || checked || unset) {   // uniform: a range's end steps, the first ones, or an overflow
+            typedef uint16_t u16x2 __attribute__((ext_vector_type(2)));
+            auto largest = [&]() -> uint32_t {
+              u16x2 top = 0;
 #pragma unroll
-            for (int kk = 0; kk < KT; kk++)
+              for (int kk = 0; kk < KT; kk++)
 #pragma unroll
-              for (int i = 0; i < 4 * NCH; i++) {
-                const uint32_t wv = ((const uint32_t*)vs[kk])[i >> 1];
-                mx = max(mx, ((i & 1) ? (wv >> 16) : wv) & 0x7fffu);
-              }
-            const float dm = xmax_groups(h_to_f((uint16_t)mx));
-            const float pc = (float)(7 - __builtin_amdgcn_readfirstlane(__builtin_amdgcn_frexp_expf(dm)));
-            if (pc < pup) {   // O and lsum are zero on the first step; otherwise an exact rescale
-              const float alpha = exp2_fast(pc - pup);
+                for (int i = 0; i < 4 * C::NVS; i++)
+                  top = __builtin_elementwise_max(top, __builtin_bit_cast(u16x2, ((const uint32_t*)vs[kk])[i] & 0x7fff7fffu));
+              return max(top[0], top[1]);
+            };
+            uint32_t mx = largest();
+            if (__builtin_expect(need_mask && __ballot(mx >= 0x7c00u) != 0, 0)) {
 #pragma unroll
               for (int x = 0; x < NB; x++) {
-                lsum[x] *= alpha;
+                const uint32_t k0 = lane_key();
+                uint32_t hit = 0;
 #pragma unroll
-                for (int j = 0; j < NJ; j++) O[x][j] *= alpha;
+                for (int i = 0; i < 4 * KT; i++) {
+                  uint32_t of_key = 0;
+#pragma unroll
+                  for (int b = 0; b < NCH; b++) {
+                    uint32_t h = half_at(i, b);
+                    asm volatile("" : "+v"(h));   // tested here alone: kept tests would not fit the registers
+                    of_key |= h >= 0x7c00u ? 1u << b : 0u;
+                  }
+                  hit |= sees(x, i, k0) ? of_key : 0u;
+                }
+                hit |= (uint32_t)__shfl_xor((int)hit, 16);
+                hit |= (uint32_t)__shfl_xor((int)hit, 32);
+                bad_blk[x] |= hit;
               }
-              pup = pc;
+#pragma unroll
+              for (int kk = 0; kk < KT; kk++)
+#pragma unroll
+                for (int i = 0; i < 4 * C::NVS; i++) {
+                  uint32_t wv = ((uint32_t*)vs[kk])[i];
+                  asm volatile("" : "+v"(wv));
+                  wv &= ((wv & 0x7fffu) >= 0x7c00u ? 0u : 0xffffu) | ((wv & 0x7fff0000u) >= 0x7c000000u ? 0u : 0xffff0000u);
+                  ((uint32_t*)vs[kk])[i] = wv;
+                }
+            }
+            if (checked || unset) {   // until every column has seen a key, or every step after an overflow
+              bool none = false;
+#pragma unroll
+              for (int x = 0; x < NB; x++) {
+                if (need_mask) {
+                  const uint32_t k0 = lane_key();
+                  mx = 0;
+#pragma unroll
+                  for (int i = 0; i < 4 * KT; i++) {
+                    uint32_t km = 0;
+#pragma unroll
+                    for (int b = 0; b < NCH; b++) km = max(km, half_at(i, b));
+                    mx = max(mx, sees(x, i, k0) ? km : 0u);
+                  }
+                }
+                const float pc = (float)(7 - __builtin_amdgcn_frexp_expf(xmax_groups(h_to_f((uint16_t)mx))));
+                none |= m[x] == -INFINITY;
+                if (m[x] != -INFINITY && pc < pup[x]) {   // O and lsum are zero on its first step; otherwise an exact rescale
+                  const float alpha = exp2_fast(pc - pup[x]);
+                  lsum[x] *= alpha;
+#pragma unroll
+                  for (int j = 0; j < NJ; j++) O[x][j] *= alpha;
+                  pup[x] = pc;
+                }
+              }
+              unset = __ballot(none) != 0;
             }
           }
         }
 #pragma unroll
         for (int x = 0; x < NB; x++) {
-          const float mref = (m[x] == -INFINITY ? 0.f : m[x]) - pup;   // every score is -inf while m is
+          const float mref = m[x] == -INFINITY ? 0.f : m[x] - pup[x];   // every score is -inf while m is
 #pragma unroll
           for (int i = 0; i < 4 * KT; i++) p[x][i] = exp2_fast(p[x][i] - mref);
 #pragma unroll
@@ -459,7 +530,7 @@ __device__ __forceinline__ void unit_wave(const PageGeom& g, const UnitGeom& u, 
         // A key some columns do not see may hold anything (a later row's value, or what an earlier owner
         // of the page left), and 0 * inf is not 0. Non-finite values of such a step stay out of its
         // products, and reach the columns that see them afterwards. (bf16 tiles: values beyond f16's
-        // range too, as their products are taken in f16. q8_0 values are finite below 8e6.)
+        // range too, as their products are taken in f16. q8_0: by its scales, above.)
         bool bad_v = false;
         auto nonfinite = [](uint32_t v) -> uint32_t {   // mask of the word's non-finite values
           if constexpr (F32) return (v & 0x7f800000u) == 0x7f800000u ? ~0u : 0u;
@@ -620,14 +691,14 @@ __device__ __forceinline__ void unit_wave(const PageGeom& g, const UnitGeom& u, 
             bases(st);
 #pragma unroll
             for (int b = 0; b < C::VR; b++) load_v(b);
+            const uint32_t k0 = lane_key();
             float see[NB][F32 ? 4 : 1];
             h8 seeh[NB];
 #pragma unroll
             for (int x = 0; x < NB; x++)
 #pragma unroll
               for (int i = 0; i < 4 * KT; i++) {
-                const uint32_t key = key0 + 16 * (i >> 2) + 4 * grp + (i & 3);
-                const bool on = key <= cpos[x] && key >= clo[x] && key < page_end << 4;
+                const bool on = sees(x, i, k0);
                 if constexpr (F32) see[x][i] = on ? 1.0f : 0.0f;
                 else seeh[x][i] = on ? (_Float16)1.0f : (_Float16)0.0f;
               }
@@ -700,6 +771,15 @@ __device__ __forceinline__ void unit_wave(const PageGeom& g, const UnitGeom& u, 
       if (!__ballot(bad)) break;
       checked = true;
     }
+    if constexpr (Q8) {
+#pragma unroll
+      for (int x = 0; x < NB; x++) {
+        if (!__builtin_expect(__ballot(bad_blk[x] != 0) != 0, 0)) continue;
+#pragma unroll
+        for (int j = 0; j < NJ; j++)
+          if (bad_blk[x] >> (j >> 1) & 1u) O[x][j] = f4{NAN, NAN, NAN, NAN};
+      }
+    }
 #pragma unroll
     for (int x = 0; x < NB; x++) lsum[x] = xsum_groups(lsum[x]);
   }
@@ -718,7 +798,7 @@ __device__ __forceinline__ void unit_wave(const PageGeom& g, const UnitGeom& u, 
 #pragma unroll
       for (int gi = 0; gi < NJ / GRP; gi++) store_dims<F>(op, gi, grp, hdv, &O[x][gi * GRP], mul);
       if (slot != NO_SLOT && grp == 0) {
-        op[hdv] = m[x] - pup;   // the reference the weights were taken against
+        op[hdv] = m[x] - pup[x];   // the reference the weights were taken against
         op[hdv + 1] = lsum[x];
       }
     }
@@ -735,7 +815,7 @@ __device__ __forceinline__ void unit_wave(const PageGeom& g, const UnitGeom& u, 
 #pragma unroll
       for (int j = 0; j < NJ; j++) *(f4*)(lx + (j * 64 + lane) * 4) = O[x][j];
       if (grp == 0) {
-        lx[NJ * 256 + hq] = m[x] - pup;
+        lx[NJ * 256 + hq] = m[x] - pup[x];
         lx[NJ * 256 + 16 + hq] = lsum[x];
       }
     }

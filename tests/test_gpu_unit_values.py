@@ -1,0 +1,58 @@
+"""The unit launch on values at the ends of the types' ranges, as each row has them when it walks its
+own keys (attend, crates/engine/model/src/forward.rs:585-807)."""
+
+import numpy as np
+import pytest
+
+from conftest import row_rel_err
+from llmario_amd.kv import Layer
+from llmario_amd.workloads import small
+from test_gpu_parity import pair, run_gpu
+from test_gpu_units import launches
+
+pytestmark = pytest.mark.gpu
+
+
+def rewrite(hc, L, seq, at, n=1, k=None, v=None):
+    """K and V of positions at .. at + n - 1 as the functions make them from what is there."""
+    import torch
+
+    kt, vt = (torch.empty((n, L.n_kv * d), device="cuda") for d in (L.hd, L.hdv))
+    hc.gather(0, [(seq, 0, n, at)], kt, vt)
+    if k:
+        k(kt)
+    if v:
+        v(vt)
+    hc.store(0, [(seq, 0, n, at)], kt, vt)
+
+
+def unit_run(hc, w, q):
+    got, kt = launches(hc, lambda: run_gpu(hc, w, q))
+    assert kt["prefill"][1] == 1 and kt["decode"][1] == 0 and kt["mixed"][1] == 0, kt
+    return got
+
+
+# q8_0 tiles: runs of drafted tokens across a tile's end, prompts at either edge of a window. 1e7 is
+# beyond an f16 scale (8.3e6); 1e6 is held, with a scale 5e5 times the other keys'.
+@pytest.mark.parametrize("geo,prior,new,window,at", [
+    ((32, 8, 128, 128), 3005, 7, 0, 3009), ((32, 32, 64, 64), 3005, 6, 0, 3010),
+    ((16, 4, 256, 256), 1000, 70, 1000, 1040), ((16, 4, 256, 256), 1000, 70, 1000, 30),
+    ((8, 8, 192, 192), 5, 90, 0, 20)])
+@pytest.mark.parametrize("bad", [float("inf"), float("-inf"), 1e7, 1e6])
+def test_a_row_on_q8_0_tiles_ignores_values_it_does_not_see(cuda, geo, prior, new, window, at, bad):
+    w = small("uq", "q8_0", Layer(*geo), prior=[prior] * 4, new=[new] * 4, window=window, seed=93)
+    hc, oc, q = pair(w)
+    base = unit_run(hc, w, q)
+    rewrite(hc, w.layer, 1, at, v=lambda v: v.fill_(bad))
+    got = unit_run(hc, w, q)
+    pos = prior + np.arange(4 * new) - new
+    sees = (np.arange(4 * new) // new == 1) & (pos >= at)
+    if window:
+        sees &= pos < at + window
+    assert 0 < sees.sum() < new
+    if bad == 1e6:   # the rows that see it make their unit run again: its other columns round anew
+        assert np.isfinite(got).all()
+        assert row_rel_err(got[~sees], base[~sees]) <= 1e-6
+    else:
+        assert np.array_equal(got[~sees], base[~sees])
+        assert not np.isfinite(got[sees]).any()
