@@ -16,7 +16,8 @@
 //   O^T[dims x cols] += V^T . P^T    16-bit: v_mfma_f32_16x16x32_f16, P as f16 hi + lo parts
 //                                    f32:    v_mfma_f32_16x16x4f32
 // with the same lazy online softmax, precision and q8_0 scheme as the decode work item
-// (decode_tile.h). One step's operands are held; a register is requested again for the next step as
+// (decode_tile.h); in the row layout Q and P have three parts of the pages' 16-bit type (24 bits, as in
+// f32; bf16 there takes P.V in bf16). One step's operands are held; a register is requested again for the next step as
 // soon as its products are issued, so every load has a whole step to arrive in (the two-tile buffers
 // of the decode item would not leave room for a second column block).
 //
@@ -81,11 +82,13 @@ struct Cfg {
   static constexpr int VR = F32 ? HDVP / 64 * 4 : Q8 ? HDVP / 64 : HDVP / 32;   // ... and V
   static constexpr int NKS = Q8 ? (8 * (HDP / 32) + 15) / 16 : 1, NVS = Q8 ? (8 * (HDVP / 32) + 15) / 16 : 1;
   static constexpr int LF = NB * (NJ * 256 + 32);           // floats of a wave's partial in LDS
+  // Q in hi + lo parts of the tile layout's type; in three of the row layout's.
+  static constexpr int QP = ROWS && !F32 ? 3 : 2;
   // Q's lo parts in LDS where they would spill: two column blocks of 256 dims (Q and O take half of
   // a wave's 512 registers, a step's operands a quarter; a spilled register's reload waits for every
-  // page load in flight: 2.4 us per step of 32 keys)
-  static constexpr bool QLDS = !ROWS && !Q8 && HDP >= 256 && NB == 2;
-  static constexpr int QF = QLDS ? NB * NC * 256 : 0;       // floats of a wave's lo parts
+  // page load in flight: 2.4 us per step of 32 keys), or of 96 in the row layout (half the registers)
+  static constexpr bool QLDS = !F32 && !Q8 && HDP == (ROWS ? 96 : 256) && NB == 2;
+  static constexpr int QF = QLDS ? (QP - 1) * NB * NC * 256 : 0;       // floats of a wave's lo parts
 };
 
 // The dims of O^T blocks GRP * gi .. of one column, times `mul`, to the row at `op`.
@@ -244,11 +247,14 @@ __device__ __forceinline__ void unit_wave(const PageGeom& g, const UnitGeom& u, 
     first_loads();
     ids(1);
     // ---- Q of the columns as the B operand of S^T = K Q^T
-    // (QP parts: f16 hi + lo; the row layout scales a column by a power of two so that its largest
-    // element is below 1, and adds a third part on bf16 pages: 22 and 24 bits of any f32 Q)
-    constexpr int QP = F == FR_BF16 ? 3 : 2, QR = C::QLDS ? 1 : QP;
+    // (QP parts: hi + lo of the tile layout's type; three in the row layout, whose Q has all its 24 bits.
+    // f16 rows: a column is scaled by a power of two so that its largest element is below 1, and each
+    // part is the rest of the one before times 2^11, with scores of its own: 24 bits of every element
+    // down to 2^-22 of the largest)
+    constexpr int QP = C::QP, QR = C::QLDS ? 1 : QP, QS = F == FR_F16 ? 3 : 1;
     MT qp[QR][NB][F32 ? 1 : NC];
-    float* const qlo = lds + w * C::QF + lane * 4;   // QLDS: 16 bytes per lane, column block and chunk
+    float* const qlo = lds + w * C::QF + lane * 4;   // QLDS: 16 bytes per lane, lo part, column block and chunk
+    auto qlo_at = [&](int p, int x, int c) -> uint4* { return (uint4*)(qlo + (((p - 1) * NB + x) * NC + c) * 256); };
     f4 qf[NB][F32 ? NC : 1];
     float qscale[NB];   // score of a column in the log2 domain per unit of its product
 #pragma unroll
@@ -299,12 +305,16 @@ __device__ __forceinline__ void unit_wave(const PageGeom& g, const UnitGeom& u, 
                 const _Float16 hh = (_Float16)xv;
                 part[p][i] = hh;
                 xv -= (float)hh;
+                if constexpr (QS > 1) xv *= 2048.f;
               }
             }
           }
 #pragma unroll
           for (int p = 0; p < QR; p++) qp[p][x][c] = part[p];
-          if constexpr (C::QLDS) *(uint4*)(qlo + (x * NC + c) * 256) = __builtin_bit_cast(uint4, part[1]);
+          if constexpr (C::QLDS) {
+#pragma unroll
+            for (int p = 1; p < QP; p++) *qlo_at(p, x, c) = __builtin_bit_cast(uint4, part[p]);
+          }
         }
       }
     }
@@ -339,11 +349,16 @@ __device__ __forceinline__ void unit_wave(const PageGeom& g, const UnitGeom& u, 
         if constexpr (C::QLDS) asm volatile("" ::: "memory");   // the lo parts are read again each step
         // ---- scores
         f4 s[NB][KT], s1[NB];   // f32: two chains (half the length, half the rounding)
+        f4 sp[QS][NB][KT];      // f16 rows: each part of Q its own (s: their sum)
 #pragma unroll
         for (int x = 0; x < NB; x++) {
           s1[x] = f4{0.f, 0.f, 0.f, 0.f};
 #pragma unroll
-          for (int kk = 0; kk < KT; kk++) s[x][kk] = f4{0.f, 0.f, 0.f, 0.f};
+          for (int kk = 0; kk < KT; kk++) {
+            s[x][kk] = f4{0.f, 0.f, 0.f, 0.f};
+#pragma unroll
+            for (int p = 0; p < QS; p++) sp[p][x][kk] = f4{0.f, 0.f, 0.f, 0.f};
+          }
         }
 #pragma unroll
         for (int c = 0; c < NC; c++) {
@@ -377,9 +392,10 @@ __device__ __forceinline__ void unit_wave(const PageGeom& g, const UnitGeom& u, 
 #pragma unroll
                 for (int x = 0; x < NB; x++) {
                   MT qv;
-                  if constexpr (C::QLDS) qv = p == 0 ? qp[0][x][c] : __builtin_bit_cast(MT, *(const uint4*)(qlo + (x * NC + c) * 256));
+                  if constexpr (C::QLDS) qv = p == 0 ? qp[0][x][c] : __builtin_bit_cast(MT, *qlo_at(p, x, c));
                   else qv = qp[p][x][c];
-                  if constexpr (BF) s[x][kk] = __builtin_amdgcn_mfma_f32_16x16x32_bf16(kc, qv, s[x][kk], 0, 0, 0);
+                  if constexpr (QS > 1) sp[p][x][kk] = __builtin_amdgcn_mfma_f32_16x16x32_f16(kc, qv, sp[p][x][kk], 0, 0, 0);
+                  else if constexpr (BF) s[x][kk] = __builtin_amdgcn_mfma_f32_16x16x32_bf16(kc, qv, s[x][kk], 0, 0, 0);
                   else s[x][kk] = __builtin_amdgcn_mfma_f32_16x16x32_f16(kc, qv, s[x][kk], 0, 0, 0);
                 }
             }
@@ -394,6 +410,16 @@ __device__ __forceinline__ void unit_wave(const PageGeom& g, const UnitGeom& u, 
         if constexpr (F32) {
 #pragma unroll
           for (int x = 0; x < NB; x++) s[x][0] += s1[x];
+        }
+        if constexpr (QS > 1) {
+          constexpr float D = 1.f / 2048.f;
+#pragma unroll
+          for (int x = 0; x < NB; x++)
+#pragma unroll
+            for (int kk = 0; kk < KT; kk++)
+#pragma unroll
+              for (int r = 0; r < 4; r++)
+                s[x][kk][r] = fmaf(fmaf(sp[2][x][kk][r], D, sp[1][x][kk][r]), D, sp[0][x][kk][r]);
         }
         // ---- online softmax (log2 domain), masks on a range's end steps only (uniform)
         const uint32_t key0 = (page0 + st * KT) << 4;
@@ -620,9 +646,9 @@ __device__ __forceinline__ void unit_wave(const PageGeom& g, const UnitGeom& u, 
           }
           load_vs();
         } else {
-          // P as f16 hi + lo parts on V in f16 (bf16 V widened), or on the bf16 row layout as three
-          // bf16 parts on V as it is
-          constexpr int PP = F == FR_BF16 ? 3 : 2;
+          // P as f16 hi + lo parts on V in f16 (bf16 tiles widened), or in the row layout as three parts of
+          // the pages' type on V as it is
+          constexpr int PP = ROWS ? 3 : 2;
           using PT = typename std::conditional<F == FR_BF16, b8, h8>::type;
           PT pp[PP][NB];
 #pragma unroll
@@ -639,6 +665,16 @@ __device__ __forceinline__ void unit_wave(const PageGeom& g, const UnitGeom& u, 
                   const uint32_t h = __builtin_bit_cast(uint32_t, __builtin_convertvector(r, bf2));
                   pw[k][i] = h;
                   r -= f2{__uint_as_float(h << 16), __uint_as_float(h & 0xffff0000u)};
+                }
+              } else if constexpr (F == FR_F16) {
+                typedef float f2 __attribute__((ext_vector_type(2)));
+                typedef _Float16 h2 __attribute__((ext_vector_type(2)));
+                f2 r = {p[x][2 * i], p[x][2 * i + 1]};
+#pragma unroll
+                for (int k = 0; k < PP; k++) {
+                  const h2 h = __builtin_convertvector(r, h2);
+                  pw[k][i] = __builtin_bit_cast(uint32_t, h);
+                  r = f2{__builtin_fmaf((float)h[0], -1.0f, r[0]), __builtin_fmaf((float)h[1], -1.0f, r[1])};
                 }
               } else {
                 split_pair(p[x][2 * i], p[x][2 * i + 1], pw[0][i], pw[1][i]);
@@ -865,7 +901,7 @@ template <int F, int HDP, int HDVP, int NB>
 constexpr int unit_wpe() {
   using C = Cfg<F, HDP, HDVP, NB>;
   constexpr int regs = C::KT * 4 * (C::KR + C::VR + (C::Q8 ? C::NKS + C::NVS : 0)) +
-                       NB * (C::NC * (F == FR_BF16 ? 12 : C::F32 ? 4 : 8) + C::NJ * 4);
+                       NB * (C::NC * (C::F32 ? 4 : C::ROWS ? 12 : 8) + C::NJ * 4);
   return regs > 190 ? 1 : NB == 1 && !C::ROWS && regs < 96 ? 4 : 2;
 }
 template <int F, int HDP, int HDVP, int NB>
@@ -924,9 +960,15 @@ bool with_instance(uint32_t kv_type, uint32_t hd, uint32_t hdv, uint32_t layout,
 }
 
 // Two column blocks where they fit the register file (past it, q8_0 pages at hd 256 spilled 270
-// registers into scratch memory: 5 rows x 6,000 keys 53 us against 28 with one block)
+// registers into scratch memory: 5 rows x 6,000 keys 53 us against 28 with one block). In the row layout,
+// whose Q and P have three parts, two blocks of 128 dims leave one wave per SIMD: two prompts of 1,500
+// tokens, 12/4 heads of 112, f16 99.1 us against 77.3 with one block; bf16, 32/8 heads of 104, 2,500 tokens
+// 397 and 312; of 96 dims, with Q's lo parts in LDS, two blocks are faster (two of 300 tokens, 32 heads of
+// 80, f16: 30.8 and 33.0).
 template <int F, int HDP, int HDVP>
-constexpr bool two_blocks() { return F == FT_F16 || F == FT_BF16 || (F == FR_F32 ? HDP < 256 : HDP < 192); }
+constexpr bool two_blocks() {
+  return F == FT_F16 || F == FT_BF16 || (F == FR_F32 ? HDP < 256 : F >= FR_F16 ? HDP < 128 : HDP < 192);
+}
 
 }  // namespace
 

@@ -56,3 +56,19 @@ def test_a_row_on_q8_0_tiles_ignores_values_it_does_not_see(cuda, geo, prior, ne
     else:
         assert np.array_equal(got[~sees], base[~sees])
         assert not np.isfinite(got[sees]).any()
+
+
+@pytest.mark.parametrize("kv", ["f16", "bf16"])
+def test_q_keeps_its_small_elements(cuda, kv):
+    """One dim of Q is 2^14 times the others where K is zero: the outputs are those of a Q without it,
+    to the rounding of the scores (|s| <= 16, sums of 80 products in f32: 2^-24 x 16 x 80^0.5 < 1e-5)."""
+    w = small("up", kv, Layer(8, 2, 80, 80), prior=[400], new=[5], seed=103)
+    hc, oc, q = pair(w)
+    L = w.layer
+    rewrite(hc, L, 0, 0, n=405, k=lambda k: k.view(-1, L.n_kv, L.hd)[:, :, 7].fill_(0.0))
+    q = np.random.default_rng(104).standard_normal(q.shape).astype(np.float32)
+    q[:, :, 7] = 0
+    base = unit_run(hc, w, q)
+    q[:, :, 7] = 2.0 ** 14
+    got = unit_run(hc, w, q)
+    assert row_rel_err(got, base) <= 1e-5
