@@ -251,7 +251,7 @@ __device__ __forceinline__ void unit_wave(const PageGeom& g, const UnitGeom& u, 
     // f16 rows: a column is scaled by a power of two so that its largest element is below 1, and each
     // part is the rest of the one before times 2^11, with scores of its own: 24 bits of every element
     // down to 2^-22 of the largest)
-    constexpr int QP = C::QP, QR = C::QLDS ? 1 : QP, QS = F == FR_F16 ? 3 : 1;
+    constexpr int QP = C::QP, QR = C::QLDS ? 1 : QP, QS = F == FR_F16 ? 3 : F == FR_BF16 ? 2 : 1;
     MT qp[QR][NB][F32 ? 1 : NC];
     float* const qlo = lds + w * C::QF + lane * 4;   // QLDS: 16 bytes per lane, lo part, column block and chunk
     auto qlo_at = [&](int p, int x, int c) -> uint4* { return (uint4*)(qlo + (((p - 1) * NB + x) * NC + c) * 256); };
@@ -305,7 +305,7 @@ __device__ __forceinline__ void unit_wave(const PageGeom& g, const UnitGeom& u, 
                 const _Float16 hh = (_Float16)xv;
                 part[p][i] = hh;
                 xv -= (float)hh;
-                if constexpr (QS > 1) xv *= 2048.f;
+                if constexpr (QS == 3) xv *= 2048.f;
               }
             }
           }
@@ -349,7 +349,9 @@ __device__ __forceinline__ void unit_wave(const PageGeom& g, const UnitGeom& u, 
         if constexpr (C::QLDS) asm volatile("" ::: "memory");   // the lo parts are read again each step
         // ---- scores
         f4 s[NB][KT], s1[NB];   // f32: two chains (half the length, half the rounding)
-        f4 sp[QS][NB][KT];      // f16 rows: each part of Q its own (s: their sum)
+        // rows: those of Q's first part and of the rest apart (f16: of each part). An infinite K makes the
+        // first infinite, as the reference's sum, or NaN, and the rest anything, which is kept finite.
+        f4 sp[QS][NB][KT];
 #pragma unroll
         for (int x = 0; x < NB; x++) {
           s1[x] = f4{0.f, 0.f, 0.f, 0.f};
@@ -394,9 +396,9 @@ __device__ __forceinline__ void unit_wave(const PageGeom& g, const UnitGeom& u, 
                   MT qv;
                   if constexpr (C::QLDS) qv = p == 0 ? qp[0][x][c] : __builtin_bit_cast(MT, *qlo_at(p, x, c));
                   else qv = qp[p][x][c];
-                  if constexpr (QS > 1) sp[p][x][kk] = __builtin_amdgcn_mfma_f32_16x16x32_f16(kc, qv, sp[p][x][kk], 0, 0, 0);
-                  else if constexpr (BF) s[x][kk] = __builtin_amdgcn_mfma_f32_16x16x32_bf16(kc, qv, s[x][kk], 0, 0, 0);
-                  else s[x][kk] = __builtin_amdgcn_mfma_f32_16x16x32_f16(kc, qv, s[x][kk], 0, 0, 0);
+                  f4& to = QS > 1 ? sp[p < QS ? p : QS - 1][x][kk] : s[x][kk];
+                  if constexpr (BF) to = __builtin_amdgcn_mfma_f32_16x16x32_bf16(kc, qv, to, 0, 0, 0);
+                  else to = __builtin_amdgcn_mfma_f32_16x16x32_f16(kc, qv, to, 0, 0, 0);
                 }
             }
           }
@@ -412,14 +414,16 @@ __device__ __forceinline__ void unit_wave(const PageGeom& g, const UnitGeom& u, 
           for (int x = 0; x < NB; x++) s[x][0] += s1[x];
         }
         if constexpr (QS > 1) {
-          constexpr float D = 1.f / 2048.f;
+          constexpr float D = QS == 3 ? 1.f / 2048.f : 1.f;
 #pragma unroll
           for (int x = 0; x < NB; x++)
 #pragma unroll
             for (int kk = 0; kk < KT; kk++)
 #pragma unroll
-              for (int r = 0; r < 4; r++)
-                s[x][kk][r] = fmaf(fmaf(sp[2][x][kk][r], D, sp[1][x][kk][r]), D, sp[0][x][kk][r]);
+              for (int r = 0; r < 4; r++) {
+                const float s0 = sp[0][x][kk][r], rest = QS == 3 ? fmaf(sp[QS - 1][x][kk][r], D, sp[1][x][kk][r]) : sp[1][x][kk][r];
+                s[x][kk][r] = fmaf(__builtin_amdgcn_fmed3f(rest, -1e30f, 1e30f), D, s0);   // (NaN too becomes finite)
+              }
         }
         // ---- online softmax (log2 domain), masks on a range's end steps only (uniform)
         const uint32_t key0 = (page0 + st * KT) << 4;
@@ -556,7 +560,8 @@ __device__ __forceinline__ void unit_wave(const PageGeom& g, const UnitGeom& u, 
         // A key some columns do not see may hold anything (a later row's value, or what an earlier owner
         // of the page left), and 0 * inf is not 0. Non-finite values of such a step stay out of its
         // products, and reach the columns that see them afterwards. (bf16 tiles: values beyond f16's
-        // range too, as their products are taken in f16. q8_0: by its scales, above.)
+        // range too, as their products are taken in f16. q8_0: by its scales, above.) The 16-bit row layout
+        // does so on every step: inf times the parts of a weight, of either sign, would be NaN.
         bool bad_v = false;
         auto nonfinite = [](uint32_t v) -> uint32_t {   // mask of the word's non-finite values
           if constexpr (F32) return (v & 0x7f800000u) == 0x7f800000u ? ~0u : 0u;
@@ -564,7 +569,7 @@ __device__ __forceinline__ void unit_wave(const PageGeom& g, const UnitGeom& u, 
           return ((v & 0x7fffu) >= E ? 0xffffu : 0u) | ((v & 0x7fff0000u) >= E << 16 ? 0xffff0000u : 0u);
         };
         if constexpr (!Q8) {
-          if (need_mask) {
+          if (need_mask || (ROWS && !F32)) {
             // the largest magnitude (two operations a word: the step waits for it)
             typedef uint16_t u16x2 __attribute__((ext_vector_type(2)));
             typename std::conditional<F32, uint32_t, u16x2>::type top = 0;
@@ -670,11 +675,13 @@ __device__ __forceinline__ void unit_wave(const PageGeom& g, const UnitGeom& u, 
                 typedef float f2 __attribute__((ext_vector_type(2)));
                 typedef _Float16 h2 __attribute__((ext_vector_type(2)));
                 f2 r = {p[x][2 * i], p[x][2 * i + 1]};
+                float m1 = -1.0f;
+                asm("" : "+v"(m1));   // the rest in one fma each, as in split_pair
 #pragma unroll
                 for (int k = 0; k < PP; k++) {
                   const h2 h = __builtin_convertvector(r, h2);
                   pw[k][i] = __builtin_bit_cast(uint32_t, h);
-                  r = f2{__builtin_fmaf((float)h[0], -1.0f, r[0]), __builtin_fmaf((float)h[1], -1.0f, r[1])};
+                  r = f2{__builtin_fmaf((float)h[0], m1, r[0]), __builtin_fmaf((float)h[1], m1, r[1])};
                 }
               } else {
                 split_pair(p[x][2 * i], p[x][2 * i + 1], pw[0][i], pw[1][i]);

@@ -72,3 +72,43 @@ def test_q_keeps_its_small_elements(cuda, kv):
     q[:, :, 7] = 2.0 ** 14
     got = unit_run(hc, w, q)
     assert row_rel_err(got, base) <= 1e-5
+
+
+@pytest.mark.parametrize("kv,geo", [("f16", (8, 2, 80, 80)), ("bf16", (4, 4, 40, 40)), ("f16", (4, 1, 200, 200)),
+                                    ("f32", (8, 4, 64, 64))])
+def test_an_infinite_value_gives_an_infinite_output(cuda, kv, geo):
+    """V of one position is +inf in some dims, -inf in others: every row that sees it, near (a masked
+    step) or far, has exactly those in these dims, and its other dims untouched."""
+    w = small("ui", kv, Layer(*geo), prior=[0], new=[300], seed=95)
+    hc, oc, q = pair(w)
+    base = unit_run(hc, w, q)
+    L, at = w.layer, 70
+    plus, minus = [d % L.hdv for d in (1, 8, 17, 33)], [d % L.hdv for d in (0, 15, 34)]
+
+    def put(v):
+        v.view(L.n_kv, L.hdv)[:, plus] = float("inf")
+        v.view(L.n_kv, L.hdv)[:, minus] = float("-inf")
+
+    rewrite(hc, L, 0, at, v=put)
+    got = unit_run(hc, w, q)
+    assert np.array_equal(got[:at], base[:at])
+    seen, rest = got[at:], [d for d in range(L.hdv) if d not in plus + minus]
+    assert (seen[:, :, plus] == np.inf).all() and (seen[:, :, minus] == -np.inf).all()
+    assert np.array_equal(seen[:, :, rest], base[at:][:, :, rest])
+
+
+@pytest.mark.parametrize("kv,geo", [("f16", (8, 2, 80, 80)), ("bf16", (8, 2, 80, 80)), ("f32", (8, 4, 64, 64))])
+def test_a_score_of_minus_infinity_takes_no_weight(cuda, kv, geo):
+    """K of one position is -inf in a dim where every q is positive: the outputs are finite, as the
+    general path's."""
+    w = small("uk", kv, Layer(*geo), prior=[100], new=[60], seed=97)
+    hc, oc, q = pair(w)
+    q = np.random.default_rng(98).standard_normal(q.shape).astype(np.float32)
+    q[:, :, 3] = np.abs(q[:, :, 3]) + 0.01
+    L = w.layer
+    rewrite(hc, L, 0, 40, k=lambda k: k.view(L.n_kv, L.hd)[:, 3].fill_(float("-inf")))
+    got = unit_run(hc, w, q)
+    hc.set_tuning(prefill_min_rows=1 << 32, decode_min_tiles=8)
+    gen = run_gpu(hc, w, q)
+    assert np.isfinite(gen).all() and np.isfinite(got).all()
+    assert row_rel_err(got, gen) <= (2e-5 if kv == "f32" else 2e-4)
