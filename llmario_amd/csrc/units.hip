@@ -321,14 +321,15 @@ __device__ __forceinline__ void unit_wave(const PageGeom& g, const UnitGeom& u, 
 
     // pup, `checked`: as decode_item's (q8_0: weight x V scale in f16 range; a product that
     // overflowed leaves O non-finite and the unit runs again with every step's scales checked), but of a
-    // column's own keys: the largest scale of the first step in which it sees one.
+    // column's own keys: the largest scale of the first step in which it sees one. Where the products are
+    // in f32's range, -8: no weight is over 1, so no weighted V leaves it.
     bool checked = false;
     uint32_t bad_blk[NB];   // q8_0: the 32-dim blocks for which a column sees a key of a non-finite V scale
     for (;;) {
       bool unset = true;    // q8_0, uniform: some column has seen no key yet
 #pragma unroll
       for (int x = 0; x < NB; x++) {
-        pup[x] = Q8 ? INFINITY : 7.0f;
+        pup[x] = Q8 ? INFINITY : F32 || F == FR_BF16 ? -8.0f : 7.0f;
         bad_blk[x] = 0;
         m[x] = -INFINITY;
         lsum[x] = 0.f;

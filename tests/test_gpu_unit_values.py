@@ -112,3 +112,16 @@ def test_a_score_of_minus_infinity_takes_no_weight(cuda, kv, geo):
     gen = run_gpu(hc, w, q)
     assert np.isfinite(gen).all() and np.isfinite(got).all()
     assert row_rel_err(got, gen) <= (2e-5 if kv == "f32" else 2e-4)
+
+
+@pytest.mark.parametrize("kv,geo", [("bf16", (8, 2, 80, 80)), ("f32", (8, 4, 64, 64))])
+def test_values_near_the_types_largest(cuda, kv, geo):
+    """V of about 1e36 (the largest is 3.4e38): no weighted value leaves the range of f32."""
+    w = small("ul", kv, Layer(*geo), prior=[200], new=[9], seed=101)
+    hc, oc, q = pair(w)
+    rewrite(hc, w.layer, 0, 0, n=209, v=lambda v: v.mul_(1e36))
+    got = unit_run(hc, w, q)
+    hc.set_tuning(prefill_min_rows=1 << 32, decode_min_tiles=8)
+    gen = run_gpu(hc, w, q)
+    assert np.isfinite(gen).all() and np.isfinite(got).all()
+    assert row_rel_err(got, gen) <= (2e-5 if kv == "f32" else 2e-4)
