@@ -187,7 +187,11 @@ bool plan_units(const PlanIn& in, PlanOut& o) {
   } else {
     const uint32_t c_cut = smallest([&](uint32_t x) {
       uint64_t n = 0;
-      for (const Block& b : blocks) n += (b.ns + x - 1) / x;
+      for (const Block& b : blocks) {
+        const uint64_t k = (b.ns + x - 1) / x;
+        if (k > (PF_MAX_PIECES - 2) * W) return false;   // pieces: a whole workgroup each but the ends
+        n += k;
+      }
       return n * in.n_kv + W <= target;
     });
     const uint32_t c_whole = smallest([&](uint32_t x) {
@@ -226,10 +230,11 @@ bool plan_units(const PlanIn& in, PlanOut& o) {
   uint32_t n_wg = 0;
   if (cut) {
     // units in order, each workgroup filled before the next; a little longer waves where the cuts'
-    // rounding would take one workgroup too many
+    // rounding would take one workgroup, or a unit one piece, too many
     for (;; c++) {
       mem.clear();
       n_wg = 0;
+      bool over = false;
       uint32_t room = 0;
       for (uint64_t i = 0; i < in.n_segs; i++)
         for (uint32_t kvh = 0; kvh < in.n_kv; kvh++)
@@ -250,14 +255,18 @@ bool plan_units(const PlanIn& in, PlanOut& o) {
                   continue;
                 }
                 n = room;
-                t1 = piece + 1 == PF_MAX_PIECES ? tiles : std::min(tiles, t + take);
+                t1 = std::min(tiles, t + take);
+              }
+              if (piece + 1 == PF_MAX_PIECES && t1 < tiles) {
+                over = true;
+                t1 = tiles;
               }
               mem.push_back(Member{b, kvh, t, t1, n, n_wg - 1, W - room, piece++});
               room -= n;
               t = t1;
             }
           }
-      if (n_wg <= wg_cap || c >= max_ns) break;
+      if ((n_wg <= wg_cap && !over) || c >= max_ns) break;
     }
   } else {
     // whole units, their waves capped at a workgroup's: those with the most waves first, so the

@@ -28,6 +28,8 @@ CASES = [
     ("bf16", (32, 32, 64, 64), [1210, 900], [7, 7], 500, 16),
     ("q8_0", (32, 32, 64, 64), [1215, 400], [7, 5], 0, 16),
     ("f16", (64, 8, 128, 128), [9000], [7], 0, 16),          # one long context: key pieces
+    ("f16", (12, 2, 128, 128), [30000], [4], 0, 16),         # few KV heads: a unit in up to 64 pieces
+    ("f16", (4, 1, 80, 80), [30000], [1], 0, 16),
     # prompts on widths without a prefill instance
     ("bf16", (16, 4, 256, 256), [1000, 0, 40], [150, 190, 1], 300, 16),
     ("f16", (64, 2, 256, 256), [60], [290], 0, 16),          # 32 query heads per KV head

@@ -100,3 +100,23 @@ def test_a_call_given_back_keeps_the_items_head_blocks():
     items, merges, units, c = plan("f16", *geo, 16, table, segs, noalloc=True)
     assert len(units) == 0 and len(items) == n * 16 * 2 and c.ng == 4
     check_plan("f16", *geo, 16, table, segs, 0, items, merges, units, c, noalloc=True)
+
+
+@pytest.mark.parametrize("kv,geo,new", [
+    ("f16", (12, 2, 128, 128), 4), ("q8_0", (12, 2, 128, 128), 4), ("f16", (8, 1, 128, 128), 4), ("bf16", (8, 1, 256, 256), 6),
+    ("f16", (4, 1, 80, 80), 1), ("bf16", (6, 2, 80, 80), 1), ("f32", (16, 2, 128, 128), 1), ("f32", (3, 3, 64, 64), 3)])
+@pytest.mark.parametrize("ctx", [8000, 32000, 130000])
+def test_few_units_share_a_long_context_evenly(kv, geo, new, ctx):
+    """One sequence, one to three KV heads: a unit runs as at most 64 pieces, no piece more than twice
+    the pages of an even share (of the pieces, or of 512 workgroups where those are fewer; a workgroup
+    of 8 waves of 4 pages at the least). Short contexts may stay on the decode items."""
+    table = contiguous_table([ctx + new], 16)
+    segs = [(0, 0, new, ctx)]
+    items, merges, units, c = plan(kv, *geo, 16, table, segs)
+    check_plan(kv, *geo, 16, table, segs, 0, items, merges, units, c)
+    assert len(units) > 0 or (ctx < 130000 and new > 1)
+    n_pages = (ctx + new + 15) // 16
+    live = [u for u in units if int(u[4]) != 0]
+    n_units = len({(int(u[1]), int(u[5])) for u in live})
+    longest = max([int(u[8]) for u in live], default=0)
+    assert longest <= 2 * max(n_pages / 64, n_pages * n_units / 512) + 32, (longest, n_pages, n_units)
