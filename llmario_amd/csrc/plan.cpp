@@ -170,7 +170,7 @@ bool plan_units(const PlanIn& in, PlanOut& o) {
   // (c_whole). Cutting has to save more than the merge launch costs.
   const uint32_t c_min = 4 / KT;
   const uint32_t slack = f32 ? 6 : 3;   // steps: the merge launch's ~4.5 us at ~1.5 us (a 16-key f32 step: 0.8 us)
-  const bool cut_ok = !in.prefill_no_split && !in.noalloc && group <= 16 && in.hdv <= 256 && in.hdv % 4 == 0;
+  const bool cut_ok = !in.prefill_no_split && group <= 16 && in.hdv <= 256 && in.hdv % 4 == 0;
   auto smallest = [&](auto&& fits) {
     uint32_t lo = (uint32_t)std::max<uint64_t>(c_min, (total + target - 1) / target), hi = std::max<uint32_t>(lo, (uint32_t)max_ns);
     while (lo < hi) {
@@ -180,7 +180,20 @@ bool plan_units(const PlanIn& in, PlanOut& o) {
     }
     return lo;
   };
-  uint32_t c;
+  // The 16-key tiles a wave of the decode items would walk (as plan_attend sizes them). Whole units that
+  // walk much more leave the device idle (an allocation-free call of 4 rows on 32,000 keys, 32/8 heads,
+  // f16: 8 workgroups, 275 us; 1,024 items 49; in pieces 39).
+  const uint32_t item_heads = in.layout == LAYOUT_ROWS ? in.rows_max_heads : 16;
+  uint64_t item_tiles = 0;
+  for (uint64_t t = 0; t < in.n_rows; t++) {
+    const uint64_t pos = (uint64_t)in.row_pos[t];
+    item_tiles += pos / 16 - key_lo(pos, in.window) / 16 + 1;
+  }
+  item_tiles *= (uint64_t)in.n_kv * ((group + item_heads - 1) / item_heads);
+  const bool mfma_items = in.layout == LAYOUT_TILES && !f32;
+  const uint64_t item_waves = mfma_items ? std::max<uint64_t>(in.decode_capacity / 2, in.n_cu) : std::max<uint64_t>(in.decode_capacity, 1);
+  const uint64_t item_walk = std::max<uint64_t>(mfma_items ? 8 : f32 && in.layout == LAYOUT_TILES ? 2 : 4, (item_tiles + item_waves - 1) / item_waves);
+  uint32_t c, c_whole = 0;
   bool cut = false;
   if (rounds) {
     c = (uint32_t)std::max<uint64_t>(c_min, (total + target - 1) / target);
@@ -194,7 +207,7 @@ bool plan_units(const PlanIn& in, PlanOut& o) {
       }
       return n * in.n_kv + W <= target;
     });
-    const uint32_t c_whole = smallest([&](uint32_t x) {
+    c_whole = smallest([&](uint32_t x) {
       uint64_t count[UNIT_MAX_WAVES + 1] = {}, wgs = 0;
       for (const Block& b : blocks) {
         const uint32_t n = (b.ns + x - 1) / x;
@@ -213,8 +226,10 @@ bool plan_units(const PlanIn& in, PlanOut& o) {
         }
       return wgs <= wg_cap;
     });
-    cut = cut_ok && c_whole > c_cut + slack;
-    c = cut ? c_cut : std::max(c_whole, (uint32_t)((max_ns + W - 1) / W));
+    c_whole = std::max(c_whole, (uint32_t)((max_ns + W - 1) / W));
+    // (an allocation-free call takes whole units while they walk little more than its items would)
+    cut = cut_ok && c_whole > c_cut + slack && !(in.noalloc && 2 * (uint64_t)c_whole * KT <= 3 * item_walk);
+    c = cut ? c_cut : c_whole;
   }
   // Members of workgroups: a unit, or a piece of one (whole 64-key tiles), with its waves.
   struct Member {
@@ -228,10 +243,38 @@ bool plan_units(const PlanIn& in, PlanOut& o) {
   };
   const uint32_t tile_steps = 4 / KT;
   uint32_t n_wg = 0;
+  // The units in several pieces, whose members are consecutive: f(first member, pieces); and the most
+  // heads of one merge, few enough for about a thousand merge waves.
+  auto for_each_cut = [&](auto&& f) {
+    for (size_t i = 0; i < mem.size();) {
+      size_t e = i + 1;
+      while (e < mem.size() && mem[e].piece != 0) e++;
+      if (e - i > 1) f(i, (uint32_t)(e - i));
+      i = e;
+    }
+  };
+  uint32_t merge_heads = 1;
+  auto set_merge_heads = [&] {
+    uint64_t cols_cut = 0;
+    for_each_cut([&](size_t i, uint32_t) { cols_cut += blocks[mem[i].block].it.n_col; });
+    merge_heads = (uint32_t)std::max<uint64_t>(1, cols_cut / 1024);
+  };
+  // what an allocation-free call has for their partials (the scratch) and for the lists (the staging)
+  auto fits_noalloc = [&]() -> bool {
+    uint64_t n_slots = 0, n_merges = 0;
+    for_each_cut([&](size_t i, uint32_t k) {
+      const PrefillItem& it = blocks[mem[i].block].it;
+      n_slots += (uint64_t)it.n_tok * k;
+      for_each_merge(it, group, k, [&](uint32_t, uint32_t, uint32_t) { n_merges++; }, merge_heads);
+    });
+    const uint64_t part = (n_slots * group * (in.hdv + 4) * 4 + 255) / 256 * 256, list = n_merges * sizeof(MergeItem);
+    return part + list <= in.noalloc_bytes && (list + 255) / 256 * 256 + ((uint64_t)n_wg + 7) * W * sizeof(UnitWave) <= in.noalloc_stage;
+  };
   if (cut) {
     // units in order, each workgroup filled before the next; a little longer waves where the cuts'
-    // rounding would take one workgroup, or a unit one piece, too many
-    for (;; c++) {
+    // rounding would take one workgroup, or a unit one piece, too many, and longer ones where an
+    // allocation-free call could not hold the partials; whole units once that gains nothing
+    for (;;) {
       mem.clear();
       n_wg = 0;
       bool over = false;
@@ -266,9 +309,20 @@ bool plan_units(const PlanIn& in, PlanOut& o) {
               t = t1;
             }
           }
-      if ((n_wg <= wg_cap && !over) || c >= max_ns) break;
+      const bool packed = n_wg <= wg_cap && !over;
+      set_merge_heads();
+      if (packed && (!in.noalloc || fits_noalloc())) break;
+      c += packed ? 1 + c / 4 : 1;
+      if (c + slack >= c_whole) {
+        cut = false;
+        c = c_whole;
+        n_wg = 0;
+        mem.clear();
+        break;
+      }
     }
-  } else {
+  }
+  if (!cut) {
     // whole units, their waves capped at a workgroup's: those with the most waves first, so the
     // workgroups fill; in rounds the longest waves first
     for (uint64_t i = 0; i < in.n_segs; i++)
@@ -312,29 +366,23 @@ bool plan_units(const PlanIn& in, PlanOut& o) {
   o.u_nb = nb;
   o.u_w = W;
   auto launch_at = [&](uint32_t wg) { return n_xcd == 1 ? wg : wg % per_xcd * n_xcd + wg / per_xcd; };
-  // partial slots and merges of the units in several pieces (their members are consecutive), the heads
-  // of a merge few enough for about a thousand merge waves
-  uint64_t cut_cols = 0;
-  for (size_t i = 0; cut && i < mem.size(); i++) cut_cols += mem[i].piece == 1 ? blocks[mem[i].block].it.n_col : 0;
-  const uint32_t merge_heads = (uint32_t)std::max<uint64_t>(1, cut_cols / 1024);
   o.uwaves.assign((size_t)per_xcd * n_xcd * W, UnitWave{});
+  // partial slots and merges
   std::vector<uint32_t> slots_of;   // per member: first slot of its unit
-  if (cut) slots_of.assign(mem.size(), NO_SLOT);
-  for (size_t i = 0; cut && i < mem.size();) {
-    size_t e = i + 1;
-    while (e < mem.size() && mem[e].piece != 0) e++;
-    const uint32_t k = (uint32_t)(e - i);
-    if (k > 1) {
+  if (cut) {
+    slots_of.assign(mem.size(), NO_SLOT);
+    for_each_cut([&](size_t i, uint32_t k) {
       const PrefillItem& it = blocks[mem[i].block].it;
       const uint32_t base = o.slots, kvh = mem[i].kvh;
-      for (size_t x = i; x < e; x++) slots_of[x] = base;
       for_each_merge(it, group, k, [&](uint32_t t, uint32_t h, uint32_t nh) {
         o.merges.push_back(MergeItem{it.row0 + t, kvh, h, base + t * k, k, nh});
       }, merge_heads);
       o.slots += it.n_tok * k;
-      for (size_t x = i; x < e; x++) mem[x].piece |= k << 16;
-    }
-    i = e;
+      for (size_t x = i; x < i + k; x++) {
+        slots_of[x] = base;
+        mem[x].piece |= k << 16;
+      }
+    });
   }
   for (size_t i = 0; i < mem.size(); i++) {
     const Member& m = mem[i];

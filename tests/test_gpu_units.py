@@ -152,3 +152,22 @@ def test_a_row_on_tiles_ignores_values_it_does_not_see(cuda, kv, geo, prior, new
     assert 0 < sees.sum() < new
     assert np.array_equal(got[~sees], base[~sees])
     assert not np.isfinite(got[sees]).any()
+
+
+@pytest.mark.parametrize("kv,geo,prior,new", [
+    ("f16", (32, 8, 128, 128), [16000], [4]), ("q8_0", (32, 8, 128, 128), [16000], [4]), ("bf16", (16, 4, 256, 256), [9000], [5]),
+    ("f16", (8, 2, 80, 80), [16000], [1]), ("f32", (32, 2, 128, 128), [9000], [1]),
+    ("f16", (32, 8, 128, 128), [2000, 1500, 1700, 1900], [6, 7, 5, 6])])
+def test_allocation_free_calls(cuda, kv, geo, prior, new):
+    """lmh_attend_noalloc through the unit launch, in pieces (one long context) and whole."""
+    import torch
+
+    w = small("ua", kv, Layer(*geo), prior=prior, new=new, seed=105)
+    hc, oc, q = pair(w)
+    ref = oc.attend(0, w.segments(), q, w.scale, w.window, THREADS)
+    qd, out = torch.from_numpy(q).cuda(), torch.full((q.shape[0], geo[0], geo[3]), float("nan"), device="cuda")
+    hc.attend_noalloc(0, w.segments(), qd, out, w.scale, w.window)
+    torch.cuda.synchronize()
+    err, diff = row_rel_err(out.cpu().numpy(), ref), row_rel_err(out.cpu().numpy(), run_gpu(hc, w, q))
+    print(f"{kv} {geo}: oracle {err:.3e}, attend {diff:.3e}")
+    assert err <= TOL[kv] and diff <= (1e-5 if kv == "f32" else 2e-4), (err, diff)

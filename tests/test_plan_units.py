@@ -120,3 +120,22 @@ def test_few_units_share_a_long_context_evenly(kv, geo, new, ctx):
     n_units = len({(int(u[1]), int(u[5])) for u in live})
     longest = max([int(u[8]) for u in live], default=0)
     assert longest <= 2 * max(n_pages / 64, n_pages * n_units / 512) + 32, (longest, n_pages, n_units)
+
+
+@pytest.mark.parametrize("kv,geo,new", [
+    ("f16", (32, 8, 128, 128), 4), ("q8_0", (32, 8, 128, 128), 4), ("f16", (12, 2, 128, 128), 4), ("bf16", (16, 4, 256, 256), 4),
+    ("f16", (8, 2, 80, 80), 1), ("f16", (8, 8, 80, 80), 1), ("f32", (64, 8, 128, 128), 1), ("bf16", (64, 4, 256, 256), 7)])
+@pytest.mark.parametrize("ctx", [9000, 32000])
+def test_allocation_free_calls_share_a_long_context_too(kv, geo, new, ctx):
+    """Pieces whose partials and merges fit the scratch (check_plan), the same as a call that may
+    allocate takes: no wave walks more than in that call's plan, or in decode items'."""
+    table = contiguous_table([ctx + new], 16)
+    segs = [(0, 0, new, ctx)]
+    longest = []
+    for noalloc in (False, True):
+        items, merges, units, c = plan(kv, *geo, 16, table, segs, noalloc=noalloc)
+        check_plan(kv, *geo, 16, table, segs, 0, items, merges, units, c, noalloc=noalloc)
+        longest.append(max((int(u[8]) for u in units if int(u[4]) != 0), default=0))
+        if noalloc:
+            assert c.slots * c.ng * (geo[3] + 4) * 4 + 256 + len(merges) * 24 <= 32 << 20
+    assert longest[1] <= 1.5 * longest[0], longest
