@@ -170,7 +170,7 @@ bool plan_units(const PlanIn& in, PlanOut& o) {
   // (c_whole). Cutting has to save more than the merge launch costs.
   const uint32_t c_min = 4 / KT;
   const uint32_t slack = f32 ? 6 : 3;   // steps: the merge launch's ~4.5 us at ~1.5 us (a 16-key f32 step: 0.8 us)
-  const bool cut_ok = !in.prefill_no_split && group <= 16 && in.hdv <= 256 && in.hdv % 4 == 0;
+  const bool cut_ok = !in.prefill_no_split && in.hdv <= 256 && in.hdv % 4 == 0;
   auto smallest = [&](auto&& fits) {
     uint32_t lo = (uint32_t)std::max<uint64_t>(c_min, (total + target - 1) / target), hi = std::max<uint32_t>(lo, (uint32_t)max_ns);
     while (lo < hi) {
@@ -362,7 +362,16 @@ bool plan_units(const PlanIn& in, PlanOut& o) {
   // A wave's record is longer than a decode item's: calls of many single rows whose list of items fits
   // the staging of an allocation-free call, and this one not, stay on the decode items.
   if (in.noalloc && (uint64_t)per_xcd * n_xcd * W * sizeof(UnitWave) > in.noalloc_stage) return false;
-  o.ng = (uint32_t)std::min<uint64_t>(group, 16);   // a partial slot holds the group's heads (pieces: group <= 16)
+  // Units that could not be cut as far as that (split settings, a full scratch, the cap on pieces) and walk
+  // much longer than the items would: the row layout's items, on the VALU, take ~20 times a unit's time
+  // per tile (22-29 us against 0.8-1.1), f32 pages' ~4 (15 against 3.4).
+  uint64_t walk = 0;
+  for (const Member& m : mem) {
+    const uint32_t ns = (pages_of(m) + KT - 1) / KT, n = std::min(m.n, ns);
+    walk = std::max<uint64_t>(walk, (uint64_t)(ns + n - 1) / n * KT);
+  }
+  if (!rounds && 2 * walk > 3 * item_walk * (mfma_items ? 1 : in.layout == LAYOUT_ROWS ? 20 : 4) + 16) return false;
+  o.ng = (uint32_t)group;   // a piece's partial slot holds the group's heads
   o.u_nb = nb;
   o.u_w = W;
   auto launch_at = [&](uint32_t wg) { return n_xcd == 1 ? wg : wg % per_xcd * n_xcd + wg / per_xcd; };

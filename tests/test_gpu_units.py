@@ -30,6 +30,9 @@ CASES = [
     ("f16", (64, 8, 128, 128), [9000], [7], 0, 16),          # one long context: key pieces
     ("f16", (12, 2, 128, 128), [30000], [4], 0, 16),         # few KV heads: a unit in up to 64 pieces
     ("f16", (4, 1, 80, 80), [30000], [1], 0, 16),
+    ("bf16", (32, 1, 80, 80), [20000, 50], [1, 2], 0, 16),   # groups wider than a unit, in pieces
+    ("f16", (142, 2, 64, 64), [20000], [3], 0, 32),
+    ("f32", (64, 2, 128, 128), [9000], [1], 0, 16),
     # prompts on widths without a prefill instance
     ("bf16", (16, 4, 256, 256), [1000, 0, 40], [150, 190, 1], 300, 16),
     ("f16", (64, 2, 256, 256), [60], [290], 0, 16),          # 32 query heads per KV head
@@ -156,7 +159,7 @@ def test_a_row_on_tiles_ignores_values_it_does_not_see(cuda, kv, geo, prior, new
 
 @pytest.mark.parametrize("kv,geo,prior,new", [
     ("f16", (32, 8, 128, 128), [16000], [4]), ("q8_0", (32, 8, 128, 128), [16000], [4]), ("bf16", (16, 4, 256, 256), [9000], [5]),
-    ("f16", (8, 2, 80, 80), [16000], [1]), ("f32", (32, 2, 128, 128), [9000], [1]),
+    ("f16", (8, 2, 80, 80), [16000], [1]), ("f32", (64, 2, 128, 128), [9000], [1]),
     ("f16", (32, 8, 128, 128), [2000, 1500, 1700, 1900], [6, 7, 5, 6])])
 def test_allocation_free_calls(cuda, kv, geo, prior, new):
     """lmh_attend_noalloc through the unit launch, in pieces (one long context) and whole."""

@@ -139,3 +139,39 @@ def test_allocation_free_calls_share_a_long_context_too(kv, geo, new, ctx):
         if noalloc:
             assert c.slots * c.ng * (geo[3] + 4) * 4 + 256 + len(merges) * 24 <= 32 << 20
     assert longest[1] <= 1.5 * longest[0], longest
+
+
+@pytest.mark.parametrize("kv,geo,new", [
+    ("bf16", (32, 1, 80, 80), 1), ("f32", (64, 2, 128, 128), 1), ("f16", (64, 2, 128, 128), 4), ("f16", (71, 1, 64, 64), 4),
+    ("f32", (71, 1, 64, 64), 1), ("f16", (128, 1, 256, 256), 3)])
+@pytest.mark.parametrize("noalloc", [False, True])
+def test_groups_wider_than_a_unit_share_a_long_context(kv, geo, new, noalloc):
+    """More heads per group than the 16 or 32 columns of a unit: the units are cut into pieces all the
+    same, their partials at their head's position of a slot of the whole group."""
+    ctx = 32000
+    table = contiguous_table([ctx + new], 16)
+    segs = [(0, 0, new, ctx)]
+    items, merges, units, c = plan(kv, *geo, 16, table, segs, noalloc=noalloc)
+    check_plan(kv, *geo, 16, table, segs, 0, items, merges, units, c, noalloc=noalloc)
+    live = [u for u in units if int(u[4]) != 0]
+    n_units = len({(int(u[1]), int(u[2]), int(u[5])) for u in live})
+    n_pages = (ctx + new + 15) // 16
+    assert live and c.ng == geo[0] // geo[1] and all(int(u[5]) + int(u[6]) <= c.ng * int(u[4]) for u in live)
+    assert max(int(u[8]) for u in live) <= 2 * max(n_pages / 64, n_pages * n_units / 512) + 32
+    if noalloc:
+        assert c.slots * c.ng * (geo[3] + 4) * 4 + 256 + len(merges) * 24 <= 32 << 20
+
+
+def test_whole_units_give_a_long_context_back():
+    """Units never cut into pieces (prefill_whole_units): a call they would leave on a few workgroups stays
+    on the decode items, one whose units fill the device does not."""
+    for new, prior, units_expected in (([4], [32000], False), ([6] * 4, [2000] * 4, True), ([1], [32000], None)):
+        kv, geo = ("f16", (32, 8, 128, 128)) if units_expected is not None else ("f32", (64, 2, 128, 128))
+        segs, start = [], 0
+        for s, (p, n) in enumerate(zip(prior, new)):
+            segs.append((s, start, n, p))
+            start += n
+        table = contiguous_table([p + n for p, n in zip(prior, new)], 16)
+        items, merges, units, c = plan(kv, *geo, 16, table, segs, prefill_whole_units=1)
+        check_plan(kv, *geo, 16, table, segs, 0, items, merges, units, c)
+        assert (len(units) > 0) == bool(units_expected) and (len(items) > 0) != bool(units_expected)
