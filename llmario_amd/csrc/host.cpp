@@ -205,6 +205,11 @@ struct DevBuf {  // grow-only device scratch
   ~DevBuf() {
     if (p) (void)hipFree(p);
   }
+  hipError_t reserve(size_t bytes) {   // exactly, before any call
+    hipError_t e = hipMalloc(&p, bytes);
+    if (e == hipSuccess) cap = bytes;
+    return e;
+  }
   hipError_t ensure(size_t bytes) {
     if (cap >= bytes) return hipSuccess;
     if (p) {
@@ -882,6 +887,16 @@ int32_t lmh_kv_create(const lmh_kv_options* o, lmh_kv** out) {
   // staging slots sized for a call's work list (decode items, merges, prefill units: 1 MiB holds
   // ~32 K decode items) and 16 block-table rows, so calls do not grow them
   if (e == hipSuccess) e = kv->up.reserve(staging_bytes(kv->bps));
+  // partials and merges of the largest unit plan of the layers (at most 32 MiB): a first call, or a longer
+  // one in the middle of serving, does not stop for a hipMalloc (first pass on a new cache: 24 x 4 drafted
+  // rows 167-217 us -> 101-135, 32 decode rows that merge 275 -> 200; creation 290 -> 330)
+  uint64_t part_bytes = 0;
+  for (const LayerLayout& y : kv->layers) {
+    if (bt >= 16 && unit_waves(kv->kv_type, y.hd, y.hdv, y.layout, 1))
+      part_bytes = std::max(part_bytes, unit_part_bytes(kv->n_cu, y.n_head / y.n_kv, y.hdv));
+  }
+  if (e == hipSuccess && part_bytes) e = kv->part_buf.reserve(std::min<uint64_t>(part_bytes, 32ull << 20));
+  if (e == hipSuccess && part_bytes) e = kv->merge_buf.reserve(256 << 10);
   // this device's copy of lmh_attend_noalloc's scratch (resolved once per device)
   if (e == hipSuccess) e = noalloc_scratch(o->device, &kv->scratch);
   if (e == hipSuccess) {

@@ -78,4 +78,11 @@ constexpr uint64_t DEFAULT_PREFILL_MIN_ROWS = 8;
 
 void plan_attend(const PlanIn& in, PlanOut& out);
 
+// Bytes that hold a unit plan's partials on a device of n_cu compute units, for a layer of this head group
+// and value width: one round of workgroups (at most two of four waves per CU), each boundary between two
+// of them inside a unit, whose piece on either side leaves a slot per token of its up to 32 columns.
+inline uint64_t unit_part_bytes(uint32_t n_cu, uint64_t group, uint64_t hdv) {
+  return 2ull * 2 * n_cu * ((32 + group - 2) / group + 1) * group * (hdv + 4) * 4;
+}
+
 }  // namespace lmh

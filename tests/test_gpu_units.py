@@ -174,3 +174,26 @@ def test_allocation_free_calls(cuda, kv, geo, prior, new):
     err, diff = row_rel_err(out.cpu().numpy(), ref), row_rel_err(out.cpu().numpy(), run_gpu(hc, w, q))
     print(f"{kv} {geo}: oracle {err:.3e}, attend {diff:.3e}")
     assert err <= TOL[kv] and diff <= (1e-5 if kv == "f32" else 2e-4), (err, diff)
+
+
+def test_first_calls_of_a_cache_allocate_nothing(cuda):
+    """The partials of a unit plan in pieces are reserved at creation: device memory stays as it was over
+    a new cache's first calls, a longer one after a shorter one among them."""
+    import gc
+    import torch
+
+    free = []
+    for again in (False, True):   # the first cache's calls load the kernels
+        w = small("uf", "f16", Layer(32, 8, 128, 128), prior=[1900 + 3 * i for i in range(24)], new=[4] * 24, seed=107)
+        hc, oc, q = pair(w)
+        qd = torch.from_numpy(q).cuda()
+        out = torch.empty(q.shape[0], 32, 128, device="cuda")
+        gc.collect()
+        torch.cuda.synchronize()
+        free = [torch.cuda.mem_get_info()[0]]
+        for n in (8, 24):
+            hc.attend(0, w.segments()[:n], qd[:4 * n], out[:4 * n], w.scale)
+            torch.cuda.synchronize()
+            free.append(torch.cuda.mem_get_info()[0])
+    print(free)
+    assert free[0] == free[1] == free[2]
