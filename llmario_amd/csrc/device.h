@@ -206,9 +206,9 @@ hipError_t launch_mixed(const PageGeom& g, const PrefillGeom& pg, const PrefillI
                         hipStream_t s, const LaunchEv& ev = {});
 // Units (units.hip) of up to 16 * nb columns (nb 1 or 2): n_wg workgroups of w waves, a UnitWave each.
 // unit_waves: the most waves of a workgroup, 0 where no instance takes the geometry (blocks of 16
-// positions or more). unit_waves_per_cu: what a CU's registers hold at once (occupancy query).
+// positions or more). unit_waves_per_cu: what a CU of the device holds at once by its registers.
 uint32_t unit_waves(uint32_t kv_type, uint32_t hd, uint32_t hdv, uint32_t layout, uint32_t nb);
-uint32_t unit_waves_per_cu(uint32_t kv_type, uint32_t hd, uint32_t hdv, uint32_t layout, uint32_t nb);
+uint32_t unit_waves_per_cu(int32_t device, uint32_t kv_type, uint32_t hd, uint32_t hdv, uint32_t layout, uint32_t nb);
 hipError_t launch_units(const PageGeom& g, const UnitGeom& u, uint32_t nb, uint32_t w, const UnitWave* waves, uint32_t n_wg,
                         const float* q, float* out, const MergeCopy& mc, hipStream_t s, const LaunchEv& ev = {});
 uint32_t prefill_wg_per_cu();     // prefill workgroups a CU holds when their LDS fits (160 KiB / this)

@@ -263,7 +263,6 @@ struct lmh_kv {
   int device = 0;
   uint32_t n_cu = 0;                        // compute units of the device
   std::vector<uint32_t> decode_capacity;    // per layer: decode items resident at once (0 = not yet asked)
-  std::vector<std::array<uint32_t, 2>> unit_res;   // per layer: unit waves a CU holds (0 = not yet asked)
   uint8_t* d_pool = nullptr;
   int32_t* d_table = nullptr;
   std::vector<int32_t> h_table;
@@ -879,7 +878,6 @@ int32_t lmh_kv_create(const lmh_kv_options* o, lmh_kv** out) {
   if (e == hipSuccess) e = hipDeviceGetAttribute(&n_cu, hipDeviceAttributeMultiprocessorCount, o->device);
   kv->n_cu = (uint32_t)std::max(n_cu, 1);
   kv->decode_capacity.assign(kv->layers.size(), 0);
-  kv->unit_res.assign(kv->layers.size(), {0, 0});
   if (e == hipSuccess) e = hipMalloc((void**)&kv->d_pool, kv->pool_blocks * kv->block_bytes);
   if (e == hipSuccess) e = hipMalloc((void**)&kv->d_table, std::max<uint64_t>(kv->h_table.size(), 1) * 4);
   if (e == hipSuccess && kv->window) e = hipMalloc((void**)&kv->d_wpool, kv->wpool_blocks * kv->wblock_bytes);
@@ -1498,12 +1496,10 @@ static int32_t attend_impl(lmh_kv* kv, uint32_t layer, const lmh_seg* segs, uint
   pin.noalloc_bytes = NOALLOC_SCRATCH_BYTES;
   pin.noalloc_stage = list_bytes(kv->up.reserved, n_rows);
   fill_kernel_facts(pin, kv->kv_type, y.hd, y.hdv, group, y.layout);
-  for (uint32_t nb = 1; nb <= 2; nb++) {
-    if (!pin.unit_w[nb - 1]) continue;
-    uint32_t& n = kv->unit_res[layer][nb - 1];
-    if (n == 0) n = unit_waves_per_cu(kv->kv_type, y.hd, y.hdv, y.layout, nb);
-    pin.unit_waves_per_cu[nb - 1] = n;
-  }
+  pin.unit_waves_per_cu = [](const PlanIn& in, uint32_t nb) {
+    return unit_waves_per_cu(in.device, in.kv_type, in.hd, in.hdv, in.layout, nb);
+  };
+  pin.device = kv->device;
   PlanOut& pl = kv->plan;
   plan_attend(pin, pl);
   const uint32_t ng = pl.ng, slots = pl.slots, pf_wg = pl.pf_wg, pf_per_wg = pl.pf_per_wg, max_pages = pl.max_pages;

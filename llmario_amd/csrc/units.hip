@@ -42,6 +42,7 @@
 #include "decode_tile.h"
 
 #include <algorithm>
+#include <atomic>
 
 namespace lmh {
 namespace {
@@ -990,18 +991,22 @@ uint32_t unit_waves(uint32_t kv_type, uint32_t hd, uint32_t hdv, uint32_t layout
   return w;
 }
 
-// Asked of the runtime once per kernel (a query takes ~10 us, which each new cache's first call paid).
-uint32_t unit_waves_per_cu(uint32_t kv_type, uint32_t hd, uint32_t hdv, uint32_t layout, uint32_t nb) {
+// Asked of the runtime once per kernel and device (a query takes ~10 us, which each new cache's first call
+// paid); a query that fails is asked again by the next call.
+uint32_t unit_waves_per_cu(int32_t device, uint32_t kv_type, uint32_t hd, uint32_t hdv, uint32_t layout, uint32_t nb) {
+  constexpr int DEVICES = 16;   // devices beyond these are asked each time
   uint32_t n = 4;
   auto ask = [&](auto f, auto a, auto b, auto nbt) {   // without LDS, 4-wave workgroups: what the registers allow
     constexpr int F = decltype(f)::value, A = decltype(a)::value, B = decltype(b)::value, NB = decltype(nbt)::value;
     if constexpr (NB == 1 || two_blocks<F, A, B>()) {
-      static const uint32_t waves = [] {
-        int blocks = 0;
-        if (hipOccupancyMaxActiveBlocksPerMultiprocessor(&blocks, unit_kernel<F, A, B, NB>, 256, 0) != hipSuccess) blocks = 0;
-        return 4 * (uint32_t)std::max(blocks, 1);
-      }();
-      n = waves;
+      static std::atomic<uint32_t> known[DEVICES];
+      const bool keep = device >= 0 && device < DEVICES;
+      if (keep && (n = known[device].load(std::memory_order_relaxed)) != 0) return;
+      int blocks = 0;
+      const bool ok = hipSetDevice(device) == hipSuccess &&
+                      hipOccupancyMaxActiveBlocksPerMultiprocessor(&blocks, unit_kernel<F, A, B, NB>, 256, 0) == hipSuccess && blocks > 0;
+      n = ok ? 4 * (uint32_t)blocks : 4;
+      if (ok && keep) known[device].store(n, std::memory_order_relaxed);
     }
   };
   with_instance(kv_type, hd, hdv, layout, [&](auto f, auto a, auto b) {
