@@ -202,21 +202,25 @@ struct Uploader {
 struct DevBuf {  // grow-only device scratch
   void* p = nullptr;
   size_t cap = 0;
+  bool own = true;   // false: inside another allocation
   ~DevBuf() {
-    if (p) (void)hipFree(p);
+    if (p && own) (void)hipFree(p);
   }
-  hipError_t reserve(size_t bytes) {   // exactly, before any call
-    hipError_t e = hipMalloc(&p, bytes);
-    if (e == hipSuccess) cap = bytes;
-    return e;
+  void lend(void* at, size_t bytes) {
+    p = at;
+    cap = bytes;
+    own = false;
   }
   hipError_t ensure(size_t bytes) {
     if (cap >= bytes) return hipSuccess;
     if (p) {
-      (void)hipDeviceSynchronize();  // in-flight work of earlier calls may still read it
-      (void)hipFree(p);
+      if (own) {
+        (void)hipDeviceSynchronize();  // in-flight work of earlier calls may still read it
+        (void)hipFree(p);
+      }
       p = nullptr;
       cap = 0;
+      own = true;
     }
     size_t c = std::max<size_t>(bytes + bytes / 4, 1 << 16);
     hipError_t e = hipMalloc(&p, c);
@@ -878,23 +882,28 @@ int32_t lmh_kv_create(const lmh_kv_options* o, lmh_kv** out) {
   if (e == hipSuccess) e = hipDeviceGetAttribute(&n_cu, hipDeviceAttributeMultiprocessorCount, o->device);
   kv->n_cu = (uint32_t)std::max(n_cu, 1);
   kv->decode_capacity.assign(kv->layers.size(), 0);
-  if (e == hipSuccess) e = hipMalloc((void**)&kv->d_pool, kv->pool_blocks * kv->block_bytes);
+  // Behind the pool, in its allocation: partials and merges of the largest unit plan of the layers (at most
+  // 32 MiB), so that a first call, or a longer one in the middle of serving, does not stop for a hipMalloc
+  // (first pass on a new cache: 24 x 4 drafted rows 167-217 us -> 101-135, 32 decode rows that merge
+  // 275 -> 200; as allocations of their own they took creation from 290 to 330).
+  uint64_t part_bytes = 0;
+  for (const LayerLayout& y : kv->layers) {
+    if (bt >= 16 && unit_waves(kv->kv_type, y.hd, y.hdv, y.layout, 1))
+      part_bytes = std::max(part_bytes, unit_part_bytes(kv->n_cu, y.n_head / y.n_kv, y.hdv));
+  }
+  part_bytes = (std::min<uint64_t>(part_bytes, 32ull << 20) + 255) / 256 * 256;
+  const uint64_t merge_bytes = part_bytes ? 256 << 10 : 0, pool_bytes = (kv->pool_blocks * kv->block_bytes + 255) / 256 * 256;
+  if (e == hipSuccess) e = hipMalloc((void**)&kv->d_pool, pool_bytes + part_bytes + merge_bytes);
+  if (e == hipSuccess && part_bytes) {
+    kv->part_buf.lend(kv->d_pool + pool_bytes, part_bytes);
+    kv->merge_buf.lend(kv->d_pool + pool_bytes + part_bytes, merge_bytes);
+  }
   if (e == hipSuccess) e = hipMalloc((void**)&kv->d_table, std::max<uint64_t>(kv->h_table.size(), 1) * 4);
   if (e == hipSuccess && kv->window) e = hipMalloc((void**)&kv->d_wpool, kv->wpool_blocks * kv->wblock_bytes);
   if (e == hipSuccess && kv->window) e = hipMalloc((void**)&kv->d_wtable, kv->h_wtable.size() * 4);
   // staging slots sized for a call's work list (decode items, merges, prefill units: 1 MiB holds
   // ~32 K decode items) and 16 block-table rows, so calls do not grow them
   if (e == hipSuccess) e = kv->up.reserve(staging_bytes(kv->bps));
-  // partials and merges of the largest unit plan of the layers (at most 32 MiB): a first call, or a longer
-  // one in the middle of serving, does not stop for a hipMalloc (first pass on a new cache: 24 x 4 drafted
-  // rows 167-217 us -> 101-135, 32 decode rows that merge 275 -> 200; creation 290 -> 330)
-  uint64_t part_bytes = 0;
-  for (const LayerLayout& y : kv->layers) {
-    if (bt >= 16 && unit_waves(kv->kv_type, y.hd, y.hdv, y.layout, 1))
-      part_bytes = std::max(part_bytes, unit_part_bytes(kv->n_cu, y.n_head / y.n_kv, y.hdv));
-  }
-  if (e == hipSuccess && part_bytes) e = kv->part_buf.reserve(std::min<uint64_t>(part_bytes, 32ull << 20));
-  if (e == hipSuccess && part_bytes) e = kv->merge_buf.reserve(256 << 10);
   // this device's copy of lmh_attend_noalloc's scratch (resolved once per device)
   if (e == hipSuccess) e = noalloc_scratch(o->device, &kv->scratch);
   if (e == hipSuccess) {
