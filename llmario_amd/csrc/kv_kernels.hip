@@ -1553,7 +1553,7 @@ hipError_t launch_snapshot(bool write, const PageGeom& g, uint32_t seq, uint32_t
     }
   }
   if ((g.kv_type == KV_F32 || (!tiles && g.kv_type != KV_Q8)) && seg_k % 4 == 0 && seg_v % 4 == 0 &&
-      stride % 4 == 0 && bb % 4 == 0 && ((uintptr_t)bytes & 3) == 0) {
+      stride % 4 == 0 && bb % 4 == 0 && ref_off % 4 == 0 && ((uintptr_t)bytes & 3) == 0) {   // (a layer's page offset is ref_off)
     const SnapGeom sg{seq, bt, k_row, v_row, bb, ref_off, seg_k, seg_v, stride};
     const bool wide = seg_k % 16 == 0 && seg_v % 16 == 0 && bb % 16 == 0 && ref_off % 16 == 0 && ((uintptr_t)bytes & 15) == 0;
     const uint32_t words = bt * std::max(k_row, v_row) / (wide ? 16 : 4), parts = (words + 2047) / 2048;
