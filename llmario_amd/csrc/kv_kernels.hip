@@ -1392,14 +1392,15 @@ __global__ __launch_bounds__(256) void snapshot_copy_kernel(PageGeom g, SnapGeom
 }
 
 // Zero whole blocks (a newly backed block reads as zeros, like the reference's anonymous
-// mappings, kv.rs:29-37). block_bytes is a multiple of 16.
+// mappings, kv.rs:29-37), in words of 16 bytes, or 2 where the blocks are no multiple of 16.
+template <typename W>
 __global__ void zero_blocks_kernel(uint8_t* pool, uint64_t block_bytes, const int32_t* blocks, uint32_t n) {
-  const uint64_t per = block_bytes / 16u;
+  const uint64_t per = block_bytes / sizeof(W);
   const uint32_t b = blockIdx.y;
   if (b >= n) return;
-  uint4* base = (uint4*)(pool + (size_t)blocks[b] * block_bytes);
+  W* base = (W*)(pool + (size_t)blocks[b] * block_bytes);
   for (uint64_t i = (uint64_t)blockIdx.x * blockDim.x + threadIdx.x; i < per; i += (uint64_t)gridDim.x * blockDim.x)
-    base[i] = make_uint4(0, 0, 0, 0);
+    base[i] = W{};
 }
 
 }  // namespace
@@ -1632,10 +1633,13 @@ hipError_t launch_zero_blocks(uint8_t* pool, uint64_t block_bytes, const int32_t
   if (n == 0) return hipSuccess;
   const uint64_t per = block_bytes / 16u;
   uint32_t gx = (uint32_t)((per + 255) / 256);
-  if (gx > 64) gx = 64;
+  gx = gx < 1 ? 1 : gx > 64 ? 64 : gx;
   for (uint32_t b0 = 0; b0 < n; b0 += 65535u) {
     const uint32_t nb = (n - b0) < 65535u ? (n - b0) : 65535u;
-    hipLaunchKernelGGL(zero_blocks_kernel, dim3(gx, nb), dim3(256), 0, s, pool, block_bytes, blocks + b0, nb);
+    if (block_bytes % 16 == 0)
+      hipLaunchKernelGGL(zero_blocks_kernel<uint4>, dim3(gx, nb), dim3(256), 0, s, pool, block_bytes, blocks + b0, nb);
+    else
+      hipLaunchKernelGGL(zero_blocks_kernel<uint16_t>, dim3(gx, nb), dim3(256), 0, s, pool, block_bytes, blocks + b0, nb);
   }
   return hipGetLastError();
 }

@@ -19,6 +19,8 @@ CASES = [
     ("f16", [(8, 2, 80, 80)] * 3 + [(4, 2, 50, 50)] * 2, 16),     # 16- and 4-byte words
     ("bf16", [(4, 2, 33, 35)] * 2, 16),                           # rows of 66 and 70 bytes: neither
     ("f16", [(1, 1, 33, 34), (1, 1, 34, 34), (1, 1, 33, 34)], 1), # rows of 68 bytes, 134 bytes into the block
+    ("f16", [(1, 1, 33, 34), (1, 1, 33, 33), (1, 1, 34, 34)], 2), # blocks of 804 bytes: unwritten slots zero to the end
+    ("bf16", [(1, 1, 33, 34)], 4), ("f32", [(1, 1, 5, 6)], 2), ("f16", [(1, 1, 1, 2)], 2),
     ("f16", [(8, 2, 64, 128), (8, 2, 64, 128)], 16), ("bf16", [(8, 2, 128, 128)] * 2, 4),
     ("q8_0", [(4, 2, 96, 32)] * 2, 16), ("f16", [(12, 4, 96, 96)] * 2, 16),
 ]
