@@ -362,6 +362,17 @@ typedef struct lmh_plan_counts {
 int32_t lmh_plan_attend(const lmh_plan_desc* d, const lmh_seg* segs, uint64_t n_segs, uint32_t* items,
                         uint64_t items_cap, uint32_t* merges, uint64_t merges_cap, uint32_t* units,
                         uint64_t units_cap, lmh_plan_counts* counts);
+/* The same for a call that runs as one unit launch (its units are in lmh_plan_attend's lists too): the
+ * wave records the kernel reads, waves_per_wg to a workgroup (an idle wave's share count is 0), and the
+ * merges, on a device whose CUs hold waves_per_cu waves of it. n_waves 0: another launch. */
+typedef struct lmh_plan_wave_counts {
+  uint64_t n_waves, n_merges;
+  uint32_t wave_words, merge_words;
+  uint32_t waves_per_wg, col_blocks, shared, ng, slots, layout;
+} lmh_plan_wave_counts;
+int32_t lmh_plan_unit_waves(const lmh_plan_desc* d, const lmh_seg* segs, uint64_t n_segs, uint32_t waves_per_cu,
+                            uint32_t* waves, uint64_t waves_cap, uint32_t* merges, uint64_t merges_cap,
+                            lmh_plan_wave_counts* counts);
 
 /* ---- request scheduler: the host side of the batch hand-off ----
  * Scheduler (crates/engine/sched/src/lib.rs:75-282) over the block pool, with Sequence

@@ -77,6 +77,11 @@ class PlanCounts(C.Structure):
                 ("max_pages", u32), ("local", u32), ("layout", u32), ("chunk", u32)]
 
 
+class PlanWaveCounts(C.Structure):
+    _fields_ = [("n_waves", u64), ("n_merges", u64), ("wave_words", u32), ("merge_words", u32), ("waves_per_wg", u32),
+                ("col_blocks", u32), ("shared", u32), ("ng", u32), ("slots", u32), ("layout", u32)]
+
+
 PRIORITY_BATCH, PRIORITY_API, PRIORITY_INTERACTIVE = 0, 1, 2
 
 
@@ -159,6 +164,7 @@ SIGNATURES = {
     "lmh_attend_noalloc": (i32, [P, u32, P, u64, P, P, C.c_float, u64, P]),
     "lmh_kv_set_tuning": (i32, [P, C.POINTER(AttendTuning)]),
     "lmh_kv_get_tuning": (i32, [P, C.POINTER(AttendTuning)]),
+    "lmh_plan_unit_waves": (i32, [C.POINTER(PlanDesc), P, u64, u32, P, u64, P, u64, C.POINTER(PlanWaveCounts)]),
     "lmh_plan_attend": (i32, [C.POINTER(PlanDesc), P, u64, P, u64, P, u64, P, u64, C.POINTER(PlanCounts)]),
     "lmh_kv_set_timing": (i32, [P, i32]),
     "lmh_kv_kernel_time": (i32, [P, u32, C.POINTER(C.c_double), C.POINTER(u64)]),

@@ -1682,12 +1682,10 @@ int32_t lmh_kv_get_tuning(const lmh_kv* kv, lmh_attend_tuning* t) {
   return LMH_OK;
 }
 
-// The planner alone on host data (no device): validates like lmh_kv_create / lmh_attend, plans as
-// lmh_attend would for a layer of this geometry, and copies the work lists out.
-int32_t lmh_plan_attend(const lmh_plan_desc* d, const lmh_seg* segs, uint64_t n_segs, uint32_t* items,
-                        uint64_t items_cap, uint32_t* merges, uint64_t merges_cap, uint32_t* units, uint64_t units_cap,
-                        lmh_plan_counts* counts) {
-  if (!d || !counts || d->abi_version != LMH_ABI_VERSION || (n_segs > 0 && !segs)) return LMH_INVALID_ARGUMENT;
+// The planner alone on host data (no device): validates like lmh_kv_create / lmh_attend and plans as
+// lmh_attend would for a layer of this geometry.
+static int32_t plan_desc(const lmh_plan_desc* d, const lmh_seg* segs, uint64_t n_segs, PlanIn& in, PlanOut& o) {
+  if (!d || d->abi_version != LMH_ABI_VERSION || (n_segs > 0 && !segs)) return LMH_INVALID_ARGUMENT;
   const uint32_t bt = d->block_tokens;
   if (d->kv_type > LMH_KV_BF16 || bt == 0 || (bt & (bt - 1)) != 0 || d->n_kv == 0 || d->n_head == 0 ||
       d->n_head % d->n_kv != 0 || d->hd == 0 || d->hdv == 0 || d->hd > MAX_HEAD_DIM || d->hdv > MAX_HEAD_DIM ||
@@ -1711,7 +1709,6 @@ int32_t lmh_plan_attend(const lmh_plan_desc* d, const lmh_seg* segs, uint64_t n_
     }
     n_rows += sg.n;
   }
-  PlanIn in;
   in.row_seq = row_seq.data();
   in.row_pos = row_pos.data();
   in.n_rows = n_rows;
@@ -1740,8 +1737,18 @@ int32_t lmh_plan_attend(const lmh_plan_desc* d, const lmh_seg* segs, uint64_t n_
   in.noalloc_stage = list_bytes(staging_bytes(in.bps), n_rows);
   in.list_units = true;
   fill_kernel_facts(in, d->kv_type, d->hd, d->hdv, d->n_head / d->n_kv, in.layout);
-  PlanOut o;
   if (n_rows > 0) plan_attend(in, o);
+  in.row_seq = in.row_pos = nullptr;   // the arrays end here
+  return LMH_OK;
+}
+
+int32_t lmh_plan_attend(const lmh_plan_desc* d, const lmh_seg* segs, uint64_t n_segs, uint32_t* items,
+                        uint64_t items_cap, uint32_t* merges, uint64_t merges_cap, uint32_t* units, uint64_t units_cap,
+                        lmh_plan_counts* counts) {
+  if (!counts) return LMH_INVALID_ARGUMENT;
+  PlanIn in;
+  PlanOut o;
+  if (const int32_t rc = plan_desc(d, segs, n_segs, in, o); rc != LMH_OK) return rc;
   counts->n_items = o.items.size();
   counts->n_merges = o.merges.size();
   counts->n_units = o.pitems.size();
@@ -1761,6 +1768,23 @@ int32_t lmh_plan_attend(const lmh_plan_desc* d, const lmh_seg* segs, uint64_t n_
   if (!o.items.empty()) std::memcpy(items, o.items.data(), o.items.size() * sizeof(DecodeItem));
   if (!o.merges.empty()) std::memcpy(merges, o.merges.data(), o.merges.size() * sizeof(MergeItem));
   if (!o.pitems.empty()) std::memcpy(units, o.pitems.data(), o.pitems.size() * sizeof(PrefillItem));
+  return LMH_OK;
+}
+
+int32_t lmh_plan_unit_waves(const lmh_plan_desc* d, const lmh_seg* segs, uint64_t n_segs, uint32_t waves_per_cu,
+                            uint32_t* waves, uint64_t waves_cap, uint32_t* merges, uint64_t merges_cap,
+                            lmh_plan_wave_counts* counts) {
+  if (!counts || waves_per_cu == 0) return LMH_INVALID_ARGUMENT;
+  PlanIn in;
+  PlanOut o;
+  in.unit_waves_given = waves_per_cu;
+  if (const int32_t rc = plan_desc(d, segs, n_segs, in, o); rc != LMH_OK) return rc;
+  const bool units = !o.uwaves.empty();
+  *counts = lmh_plan_wave_counts{o.uwaves.size(), units ? o.merges.size() : 0, sizeof(UnitWave) / 4, sizeof(MergeItem) / 4,
+                                 o.u_w, o.u_nb, o.u_shared ? 1u : 0u, o.ng, o.slots, in.layout};
+  if (counts->n_waves > waves_cap || counts->n_merges > merges_cap) return LMH_INVALID_ARGUMENT;
+  if (counts->n_waves) std::memcpy(waves, o.uwaves.data(), o.uwaves.size() * sizeof(UnitWave));
+  if (counts->n_merges) std::memcpy(merges, o.merges.data(), o.merges.size() * sizeof(MergeItem));
   return LMH_OK;
 }
 

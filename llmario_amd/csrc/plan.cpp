@@ -157,7 +157,7 @@ bool plan_units(const PlanIn& in, PlanOut& o) {
   const uint64_t n_units = (uint64_t)blocks.size() * in.n_kv;
   // Workgroups of the most waves share the longest units; where most units have a wave of their own
   // anyway, smaller ones leave a CU's waves to finish and start independently.
-  const uint32_t w_max = in.unit_w[nb - 1], per_cu = std::max(in.unit_waves_per_cu ? in.unit_waves_per_cu(in, nb) : 8u, w_max);
+  const uint32_t w_max = in.unit_w[nb - 1], per_cu = std::max(in.unit_waves_per_cu ? in.unit_waves_per_cu(in, nb) : in.unit_waves_given, w_max);
   const uint32_t W = 2 * n_units > (uint64_t)in.n_cu * per_cu ? std::min(4u, w_max) : w_max;
   const uint64_t wg_cap = (uint64_t)in.n_cu * (per_cu / W), target = wg_cap * W;
   // More units than the device holds waves (or nearly, of very uneven lengths): several rounds.

@@ -49,8 +49,9 @@ struct PlanIn {
   bool local_merge_ok = false;      // f32 decode: split rows may merge inside their workgroup
   bool mfma_local_ok = false;       // matrix-core decode: the same, for rows split at most 4 ways
   uint32_t unit_w[2] = {0, 0};      // most waves per workgroup of the unit launch of 16 / 32 columns (0: no instance)
-  uint32_t (*unit_waves_per_cu)(const PlanIn& in, uint32_t nb) = nullptr;   // its waves a CU holds at once (null: 8),
-                                    // asked only once a call's segments are taken: it may query the device
+  uint32_t (*unit_waves_per_cu)(const PlanIn& in, uint32_t nb) = nullptr;   // its waves a CU holds at once, asked
+                                    // only once a call's segments are taken: it may query the device
+  uint32_t unit_waves_given = 8;    // the same where that is null
   int32_t device = 0;
   uint64_t noalloc_stage = ~0ull;   // noalloc: bytes of work list that fit the staging reserved at creation
   bool list_units = false;          // list the unit launch's units in pitems too (lmh_plan_attend)

@@ -4,9 +4,14 @@ none), layout, segment lengths, head group, block size, split settings. Every pl
 cover each row's keys once (check_plan: attend's ranges, crates/engine/model/src/forward.rs:585-807);
 the GPU tests compare the two routes' outputs."""
 
+import ctypes as C
+from types import SimpleNamespace
+
+import numpy as np
 import pytest
 
-from test_plan import check_plan, contiguous_table, plan
+from llmario_amd import _native as N
+from test_plan import KV, NO_SLOT, check_plan, contiguous_table, plan
 
 # kv, (n_head, n_kv, hd, hdv), block, prior, new, options, expected: "units", "items" (decode items
 # alone) or "prefill" (prefill units, beside decode items if the call has decode rows)
@@ -175,3 +180,77 @@ def test_whole_units_give_a_long_context_back():
         items, merges, units, c = plan(kv, *geo, 16, table, segs, prefill_whole_units=1)
         check_plan(kv, *geo, 16, table, segs, 0, items, merges, units, c)
         assert (len(units) > 0) == bool(units_expected) and (len(items) > 0) != bool(units_expected)
+
+
+def wave_plan(kv, n_head, n_kv, hd, hdv, bt, table, segs, window, n_cu, per_cu, noalloc):
+    n_seqs, bps = table.shape
+    tab = np.ascontiguousarray(table, dtype=np.int32)
+    d = N.PlanDesc(N.ABI_VERSION, KV[kv], n_head, n_kv, hd, hdv, bt, n_cu, 0, n_seqs, bps, tab.ctypes.data_as(C.c_void_p),
+                   window, 0.1, int(noalloc), N.AttendTuning(N.ABI_VERSION, 0, 0, 0, 0, 0, 0, 0))
+    arr = (N.Seg * len(segs))(*[N.Seg(*s) for s in segs])
+    c = N.PlanWaveCounts()
+    args = (C.byref(d), arr, len(segs), per_cu)
+    rc = N.lib().lmh_plan_unit_waves(*args, None, 0, None, 0, C.byref(c))
+    waves = np.zeros((c.n_waves, c.wave_words), np.uint32)
+    merges = np.zeros((c.n_merges, c.merge_words), np.uint32)
+    if rc != N.OK:
+        rc = N.lib().lmh_plan_unit_waves(*args, waves.ctypes.data_as(C.c_void_p), c.n_waves,
+                                         merges.ctypes.data_as(C.c_void_p), c.n_merges, C.byref(c))
+    assert rc == N.OK
+    return waves, merges, c
+
+
+WAVE_CALLS = [(f[0], f[1], f[2], f[3], f[4]) for f in FORMS if f[6] == "units"] + [
+    ("f16", (64, 8, 128, 128), 16, [9000], [7]), ("f16", (12, 2, 128, 128), 32, [30000], [4]), ("f32", (64, 2, 128, 128), 16, [9000, 5], [1, 9]),
+    ("bf16", (32, 1, 80, 80), 16, [20000, 50], [1, 2]), ("q8_0", (32, 8, 128, 128), 16, [3000, 1700, 800, 40], [4, 7, 2, 5]),
+    ("bf16", (16, 4, 256, 256), 64, [10, 700], [1500, 333]), ("f16", (32, 32, 80, 80), 16, [700 * i for i in range(9)], [1] * 8 + [120]),
+]
+
+
+@pytest.mark.parametrize("kv,geo,bt,prior,new", WAVE_CALLS,
+                         ids=[f"{f[0]}-{'x'.join(map(str, f[1]))}-{'_'.join(map(str, f[4]))}" for f in WAVE_CALLS])
+@pytest.mark.parametrize("window", [0, 333])
+def test_wave_records(kv, geo, bt, prior, new, window):
+    """The records a unit launch reads, over device sizes and occupancies: a unit's (or piece's) waves are
+    consecutive in one workgroup and share its pages in order, each a whole number of steps but the last,
+    with the block ids of the first two; put together they are a plan that covers every row once."""
+    segs, start = [], 0
+    for s, (p, n) in enumerate(zip(prior, new)):
+        segs.append((s, start, n, p))
+        start += n
+    table = contiguous_table([p + n for p, n in zip(prior, new)], bt)
+    step = 1 if kv == "f32" else 2
+    for n_cu, per_cu in ((256, 4), (256, 8), (256, 12), (256, 16), (80, 8), (12, 8), (5, 4)):
+        for noalloc in (False, True):
+            waves, merges, c = wave_plan(kv, *geo, bt, table, segs, window, n_cu, per_cu, noalloc)
+            if not len(waves):
+                continue   # given back to the items
+            W, units, at = c.waves_per_wg, [], 0
+            assert len(waves) % W == 0
+            while at < len(waves):
+                seq, row0, pos0, page0, n_pages, slot, b0, b1, head, cols = (int(x) for x in waves[at])
+                n = cols >> 16 & 0xFF
+                if n == 0:
+                    assert not waves[at].any()
+                    at += 1
+                    continue
+                assert at // W == (at + n - 1) // W and (n == 1 or c.shared)
+                page = page0
+                for j in range(n):
+                    r = [int(x) for x in waves[at + j]]
+                    assert (r[0], r[1], r[2], r[5], r[8]) == (seq, row0, pos0, slot, head)
+                    assert r[9] == (cols & ~0xFF00) | j << 8
+                    assert r[3] == page and r[4] > 0 and (j + 1 == n or r[4] % step == 0)
+                    assert r[6] == table[seq, page * 16 // bt] and r[7] == table[seq, min(page + 1, page + r[4] - 1) * 16 // bt]
+                    page += r[4]
+                kvh, c_off, n_col, k = head & 0xFFFF, head >> 16, cols & 0xFF, cols >> 24
+                assert n_col <= 16 * c.col_blocks and (k > 1) == (slot != NO_SLOT)
+                n_tok = (c_off + n_col - 1) // (geo[0] // geo[1]) + 1
+                total = page - page0
+                units.append([seq, kvh, row0, pos0, n_tok, c_off, n_col, page0, total, slot, k, 0] +
+                             [int(table[seq, (page0 + min(b, total - 1)) * 16 // bt]) for b in range(8)])
+                at += n
+            counts = SimpleNamespace(ng=c.ng, slots=c.slots, pf_wg=len(units), pf_per_wg=1, max_pages=1 << 30, local=0,
+                                     layout=c.layout, chunk=0)
+            check_plan(kv, *geo, bt, table, segs, window, np.zeros((0, 8), np.uint32), merges, np.array(units), counts,
+                       noalloc=noalloc)
