@@ -4,10 +4,12 @@ own keys (attend, crates/engine/model/src/forward.rs:585-807)."""
 import numpy as np
 import pytest
 
-from conftest import row_rel_err
+from conftest import TOL, row_rel_err
 from llmario_amd.kv import Layer
 from llmario_amd.workloads import small
-from test_gpu_parity import pair, run_gpu
+from test_gpu_cancelling import build
+from test_gpu_parity import THREADS, pair, run_gpu
+from test_gpu_q8_range import PROFILES
 from test_gpu_units import launches
 
 pytestmark = pytest.mark.gpu
@@ -125,3 +127,24 @@ def test_values_near_the_types_largest(cuda, kv, geo):
     gen = run_gpu(hc, w, q)
     assert np.isfinite(gen).all() and np.isfinite(got).all()
     assert row_rel_err(got, gen) <= (2e-5 if kv == "f32" else 2e-4)
+
+
+@pytest.mark.parametrize("geo,prior,new", [
+    ((32, 8, 128, 128), [3000, 1500, 2700, 1900], [6, 7, 5, 6]), ((16, 8, 128, 128), [2900, 2500, 1400, 700], [7, 6, 7, 7]),
+    ((32, 32, 64, 64), [3000, 1200], [6, 7]), ((8, 8, 192, 192), [100, 1400], [140, 33]), ((16, 4, 256, 256), [0, 1000], [131, 90])])
+@pytest.mark.parametrize("profile", list(PROFILES))
+def test_q8_0_scales_over_their_range(cuda, geo, prior, new, profile):
+    """V blocks whose scales span f16's range, rising or falling along the sequence: a step's products can
+    overflow what the first set, and the unit runs again (test_gpu_q8_range, for the decode items)."""
+    import torch
+
+    layer = Layer(*geo)
+    hc, oc, segs, n_rows, rng = build("q8_0", layer, prior, new, 61, v_scale=PROFILES[profile])
+    q = rng.standard_normal((n_rows, layer.n_head, layer.hd)).astype(np.float32)
+    out = torch.full((n_rows, layer.n_head, layer.hdv), float("nan"), device="cuda")
+    _, kt = launches(hc, lambda: hc.attend(0, segs, torch.from_numpy(q).cuda(), out, layer.hd ** -0.5))
+    assert kt["prefill"][1] == 1 and kt["decode"][1] == 0 and kt["mixed"][1] == 0, kt
+    got, ref = out.cpu().numpy(), oc.attend(0, segs, q, layer.hd ** -0.5, 0, THREADS)
+    err = row_rel_err(got, ref)
+    print(f"{geo} {profile}: {err:.3e}")
+    assert bool(np.isfinite(got).all()) and err <= TOL["q8_0"], err

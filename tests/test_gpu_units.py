@@ -51,6 +51,15 @@ CASES = [
     ("bf16", (4, 1, 200, 200), [700], [9], 0, 16),
     ("f16", (8, 2, 256, 128), [31, 32], [1, 1], 0, 16),
     ("f16", (4, 4, 8, 8), [37], [20], 0, 16),
+    # row-layout widths inside an instance's
+    ("f16", (4, 2, 160, 160), [300, 9], [45, 1], 0, 16),
+    ("bf16", (4, 2, 160, 144), [300, 9], [45, 1], 0, 32),
+    ("bf16", (16, 4, 104, 104), [500], [40], 0, 16),
+    ("bf16", (4, 1, 120, 128), [1900, 30], [1, 3], 200, 16),
+    ("f16", (8, 2, 256, 200), [90], [30], 0, 16),
+    # more units than the device holds waves: several rounds, the longest first
+    ("bf16", (16, 4, 256, 256), [0, 300], [1500, 900], 200, 16),
+    ("f32", (8, 8, 64, 64), [0, 30], [4200, 4100], 64, 16),
     # f32 pages
     ("f32", (8, 8, 64, 64), [0, 255], [70, 1], 0, 16),
     ("f32", (16, 2, 128, 128), [600, 900, 15], [1, 1, 1], 0, 16),
@@ -58,6 +67,14 @@ CASES = [
     ("f32", (12, 4, 96, 96), [3000], [1], 0, 16),            # key pieces
     ("f32", (4, 2, 100, 36), [50], [31], 0, 16),
 ]
+
+
+# every instance the library compiles: (page type, hd, hdv, 16-column blocks)
+TILES = [(d, d) for d in (32, 64, 96, 128, 192, 256)] + [(192, 128)]
+INSTANCES = [(kv, hd, hdv, nb) for kv in ("f16", "bf16") for hd, hdv in TILES for nb in (1, 2)]
+INSTANCES += [("q8_0", d, d, nb) for d, nb in ((64, 1), (64, 2), (128, 1), (128, 2), (192, 1), (256, 1))]
+INSTANCES += [(kv, d, d, nb) for kv in ("f16", "bf16") for d, nb in ((56, 1), (56, 2), (88, 1), (88, 2), (120, 1), (184, 1), (248, 1))]
+INSTANCES += [("f32", d, d, nb) for d, nb in ((64, 1), (64, 2), (128, 1), (128, 2), (256, 1))]
 
 
 def launches(hc, f):
@@ -197,3 +214,23 @@ def test_first_calls_of_a_cache_allocate_nothing(cuda):
             free.append(torch.cuda.mem_get_info()[0])
     print(free)
     assert free[0] == free[1] == free[2]
+
+
+@pytest.mark.parametrize("kv,hd,hdv,nb", INSTANCES, ids=[f"{i[0]}-{i[1]}x{i[2]}-{16 * i[3]}cols" for i in INSTANCES])
+def test_every_instance(cuda, kv, hd, hdv, nb):
+    """Runs of 7 rows on 14 or 28 columns of 8 KV heads (tile widths: long enough to be taken)."""
+    from test_plan import contiguous_table
+    from test_plan_units import wave_plan
+
+    tiles = kv == "q8_0" or (kv != "f32" and (hd, hdv) in TILES)
+    prior, geo = 5000 if tiles else 700, (16 * nb, 8, hd, hdv)
+    w = small("ue", kv, Layer(*geo), prior=[prior, 33], new=[7, 7], seed=109)
+    waves, merges, c = wave_plan(kv, *geo, 16, contiguous_table([prior + 7, 40], 16), w.segments(), 0, 256, 8, False)
+    assert len(waves) and c.col_blocks == nb
+    hc, oc, q = pair(w)
+    q = np.random.default_rng(110).standard_normal(q.shape).astype(np.float32)
+    got, kt = launches(hc, lambda: run_gpu(hc, w, q))
+    assert kt["prefill"][1] == 1 and kt["decode"][1] == 0 and kt["mixed"][1] == 0, kt
+    err = row_rel_err(got, oc.attend(0, w.segments(), q, w.scale, w.window, THREADS))
+    print(f"{kv} {geo}: {err:.3e}")
+    assert err <= TOL[kv], err
