@@ -323,14 +323,16 @@ __device__ __forceinline__ void unit_wave(const PageGeom& g, const UnitGeom& u, 
     // pup, `checked`: as decode_item's (q8_0: weight x V scale in f16 range; a product that
     // overflowed leaves O non-finite and the unit runs again with every step's scales checked), but of a
     // column's own keys: the largest scale of the first step in which it sees one. Where the products are
-    // in f32's range, -8: no weight is over 1, so no weighted V leaves it.
+    // in f32's range, 0, and the weights times 2^-8 (of every wave and piece alike): none is over 1, so no
+    // weighted V leaves it. (A shift in the exponent would cost its argument the bits it grows by.)
+    constexpr bool UNIT_P = F32 || F == FR_BF16;
     bool checked = false;
     uint32_t bad_blk[NB];   // q8_0: the 32-dim blocks for which a column sees a key of a non-finite V scale
     for (;;) {
       bool unset = true;    // q8_0, uniform: some column has seen no key yet
 #pragma unroll
       for (int x = 0; x < NB; x++) {
-        pup[x] = Q8 ? INFINITY : F32 || F == FR_BF16 ? -8.0f : 7.0f;
+        pup[x] = Q8 ? INFINITY : UNIT_P ? 0.0f : 7.0f;
         bad_blk[x] = 0;
         m[x] = -INFINITY;
         lsum[x] = 0.f;
@@ -554,7 +556,7 @@ __device__ __forceinline__ void unit_wave(const PageGeom& g, const UnitGeom& u, 
         for (int x = 0; x < NB; x++) {
           const float mref = m[x] == -INFINITY ? 0.f : m[x] - pup[x];   // every score is -inf while m is
 #pragma unroll
-          for (int i = 0; i < 4 * KT; i++) p[x][i] = exp2_fast(p[x][i] - mref);
+          for (int i = 0; i < 4 * KT; i++) p[x][i] = exp2_fast(p[x][i] - mref) * (UNIT_P ? 0x1p-8f : 1.0f);
 #pragma unroll
           for (int kk = 0; kk < KT; kk++)
             lsum[x] += (p[x][4 * kk] + p[x][4 * kk + 1]) + (p[x][4 * kk + 2] + p[x][4 * kk + 3]);
