@@ -882,19 +882,22 @@ int32_t lmh_kv_create(const lmh_kv_options* o, lmh_kv** out) {
   if (e == hipSuccess) e = hipDeviceGetAttribute(&n_cu, hipDeviceAttributeMultiprocessorCount, o->device);
   kv->n_cu = (uint32_t)std::max(n_cu, 1);
   kv->decode_capacity.assign(kv->layers.size(), 0);
-  // Behind the pool, in its allocation: partials and merges of the largest unit plan of the layers (at most
-  // 32 MiB), so that a first call, or a longer one in the middle of serving, does not stop for a hipMalloc
-  // (first pass on a new cache: 24 x 4 drafted rows 167-217 us -> 101-135, 32 decode rows that merge
-  // 275 -> 200; as allocations of their own they took creation from 290 to 330).
+  // Behind the pool, in its allocation: partials and merges of the largest unit plan of the layers, so that
+  // a first call, or a longer one in the middle of serving, does not stop for a hipMalloc (first pass on a
+  // new cache: 24 x 4 drafted rows 167-217 us -> 101-135, 32 decode rows that merge 275 -> 200; as
+  // allocations of their own they took creation from 290 to 330). At most 32 MiB, and a quarter of the pool:
+  // a small cache's contexts leave few pieces, and allocating more than it asks for takes longer (a pool of
+  // 1 MB with 9 MB behind it: 490 -> 880 us).
   uint64_t part_bytes = 0;
   for (const LayerLayout& y : kv->layers) {
     if (bt >= 16 && unit_waves(kv->kv_type, y.hd, y.hdv, y.layout, 1))
       part_bytes = std::max(part_bytes, unit_part_bytes(kv->n_cu, y.n_head / y.n_kv, y.hdv));
   }
-  part_bytes = (std::min<uint64_t>(part_bytes, 32ull << 20) + 255) / 256 * 256;
-  const uint64_t merge_bytes = part_bytes ? 256 << 10 : 0, pool_bytes = (kv->pool_blocks * kv->block_bytes + 255) / 256 * 256;
+  const uint64_t pool_bytes = (kv->pool_blocks * kv->block_bytes + 255) / 256 * 256;
+  part_bytes = std::min<uint64_t>({part_bytes, 32ull << 20, pool_bytes / 4}) / 256 * 256;
+  const uint64_t merge_bytes = std::min<uint64_t>(part_bytes / 8, 256 << 10) / 256 * 256;
   if (e == hipSuccess) e = hipMalloc((void**)&kv->d_pool, pool_bytes + part_bytes + merge_bytes);
-  if (e == hipSuccess && part_bytes) {
+  if (e == hipSuccess && merge_bytes) {
     kv->part_buf.lend(kv->d_pool + pool_bytes, part_bytes);
     kv->merge_buf.lend(kv->d_pool + pool_bytes + part_bytes, merge_bytes);
   }
