@@ -242,8 +242,11 @@ int32_t lmh_qk_rope_store(lmh_kv* kv, uint32_t layer, const lmh_seg* segs, uint6
  * accumulation. q is [n_rows][n_head][hd] f32, out is [n_rows][n_head][hdv] f32 (device).
  * Decode rows, split-K over pages and prefill tiles are packed into one work list: segments of at
  * least prefill_min_rows rows on f16, bf16 or q8_0 pages of head width 64 or 128 (hd = hdv) run on
- * the matrix-core prefill kernel (Metal's attn_prefill_hd{64,128}[_q8_0], backend.rs:563-569); the
- * other rows on the decode kernels. A stream under graph capture is refused with LMH_UNSUPPORTED
+ * the matrix-core prefill kernel (Metal's attn_prefill_hd{64,128}[_q8_0], backend.rs:563-569); calls
+ * without such a segment whose rows share keys (runs of drafted tokens, prompts of other widths), or
+ * whose pages the matrix-core decode kernel does not read (f16 / bf16 widths that are multiples of 8,
+ * up to 256, in a row layout; f32 pages of wide groups), run as one unit launch where that is faster;
+ * the other rows on the decode kernels. A stream under graph capture is refused with LMH_UNSUPPORTED
  * before anything is enqueued: the call's work list sits in a staging slot that later calls reuse,
  * which a replayed graph would read. */
 int32_t lmh_attend(lmh_kv* kv, uint32_t layer, const lmh_seg* segs, uint64_t n_segs, const float* q,
@@ -258,7 +261,7 @@ int32_t lmh_attend(lmh_kv* kv, uint32_t layer, const lmh_seg* segs, uint64_t n_s
  * process ends (its address is resolved once per device when a handle is created there): the
  * split count is capped to what it holds, and a call that still needs more split-K scratch, or
  * whose work list exceeds the staging capacity reserved at lmh_kv_create (1 MiB per slot: ~32 K
- * decode items), fails with LMH_INVALID_ARGUMENT and a message naming both sizes. Nothing in the
+ * decode items, or ~26 K waves of a unit launch, past which single rows run as items), fails with LMH_INVALID_ARGUMENT and a message naming both sizes. Nothing in the
  * scratch must start at zero (every partial is written before it is read). Every call on one GPU
  * shares its array, which keeps the last call's contents: calls that overlap on one GPU (other
  * streams or other handles on the same device) race; issue them in order on one stream. The
@@ -283,7 +286,8 @@ int32_t lmh_attend_noalloc(lmh_kv* kv, uint32_t layer, const lmh_seg* segs, uint
  *     row-layout layers; 1 .. 64).
  *   prefill_whole_units: 1 = prefill units always run whole; 0 (default) = when whole units would
  *     leave the device unbalanced (few, long units), their key ranges are cut into pieces spread over
- *     the workgroups, whose partial results a merge launch combines (heads per KV group <= 16).
+ *     the workgroups, whose partial results a merge launch combines (heads per KV group <= 16; in a
+ *     unit launch any).
  *   prefill_q_split: how the f16 / bf16 prefill launch takes a Q with bits below the page type
  *     (Q as f16 hi + lo parts either way, results within the same bound): 1 = the launch for
  *     exact Q, whose units with such bits run two passes of half their columns; 2 = the launch
@@ -312,7 +316,7 @@ int32_t lmh_kv_get_tuning(const lmh_kv* kv, lmh_attend_tuning* t);
  * lmh_kv_kernel_time returns the accumulated milliseconds and launch count of one kernel kind
  * since its last read, and resets them (it waits for the recorded events). */
 #define LMH_KERNEL_DECODE 0u
-#define LMH_KERNEL_PREFILL 1u
+#define LMH_KERNEL_PREFILL 1u    /* the prefill launch, or a unit launch (of decode rows too) */
 #define LMH_KERNEL_MERGE 2u
 #define LMH_KERNEL_ROPE_STORE 3u /* lmh_qk_rope_store's kernel */
 #define LMH_KERNEL_SNAPSHOT 4u   /* lmh_kv_write_seq / lmh_kv_read_seq kernels */

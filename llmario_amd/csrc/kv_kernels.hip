@@ -780,8 +780,9 @@ __device__ inline uint32_t pack16x2(float a, float b) {
 }
 
 // An aligned run of 4 tokens when hd == hdv == HD (64, 128, 256) and every rotated
-// pair sits in one lane (Normal pairs; Neox over all HD dims): the same results as
-// rope_tokens<HD / 64, 4>, with the work counted in slots of two heads of one kind (Q, K or V) for
+// pair sits in one lane (Normal pairs; Neox over all HD dims): what rope_tokens<HD / 64, 4> computes
+// (the same bits without a norm; a norm's sum of squares runs over 8 lanes here and 64 there, so its
+// last bit may differ), with the work counted in slots of two heads of one kind (Q, K or V) for
 // the run's four tokens, so every lane of a wave runs the same code, and every access 8 or 16
 // bytes wide.
 //   Q / K slot: lane L holds row (head 2s + (L >> 3 & 1), token L >> 4), the float4s

@@ -17,20 +17,22 @@
 //                                    f32:    v_mfma_f32_16x16x4f32
 // with the same lazy online softmax, precision and q8_0 scheme as the decode work item
 // (decode_tile.h); in the row layout Q and P have three parts of the pages' 16-bit type (24 bits, as in
-// f32; bf16 there takes P.V in bf16). One step's operands are held; a register is requested again for the next step as
-// soon as its products are issued, so every load has a whole step to arrive in (the two-tile buffers
-// of the decode item would not leave room for a second column block).
+// f32; bf16 there takes P.V in bf16). One step's operands are held; a register is requested again for the
+// next step as soon as its products are issued, so every load has a whole step to arrive in (the two-tile
+// buffers of the decode item would not leave room for a second column block).
 //
 // Measured, one step of lmh_attend, against a decode item per row (before; the row layout's and f32
 // pages' on the VALU): 24 sequences x 4 rows on 512 .. 4,096 keys (32/8 heads, hd 128, bf16, 190 MB of
-// pages): 98.5 -> 41.5 us (5.9 TB/s at four times the contexts: bound by HBM, the rest start-up and the
-// cut units' merge); hd 256 prompts of 600 and 800 tokens, window 1,024: 225 -> 62 us (57 before
-// non-finite V of a masked key was kept out: the masked steps wait for V to test it), two of 2,048:
-// 410 TFLOP/s (bound by the matrix cores and one wave's latency per SIMD); hd 80, 32 heads of their own
-// K/V, 8 decode rows and a 120-token chunk: 1,038 -> 30 us (decode rows alone at 8,000 keys: 5.0 TB/s);
-// f32 prompts of 450 and 390 tokens, hd 64: 102 -> 23 us. The row layout's loads are ordinary ones:
-// a row's lines are touched by several lanes' loads, and as streaming loads they were fetched again
-// for each (8,000 keys at hd 80: 200 -> 140 us).
+// pages): 98.5 -> 42 us, 36.6 of them this kernel (202 MB read at 5.5 TB/s, 5.9 at four times the contexts:
+// bound by HBM) and 4.4 the cut units' merge; hd 256 prompts of 600 and 800 tokens, window 1,024: 225 -> 62 us
+// (57 before non-finite V of a masked key was kept out: the masked steps wait for V to test it), bound by the
+// chain of one wave per SIMD's steps and a second, partly filled round of workgroups (waves resident 62 % of
+// the time, issuing VALU 25 % and in the matrix pipe 12 %), two of 2,048: 410 TFLOP/s; hd 80, 32 heads of
+// their own K/V, 8 decode rows and a 120-token chunk: 1,038 -> 30 us (23.5 + merge 4.1; 85 MB; decode rows
+// alone at 8,000 keys: 5.0 TB/s); f32 prompts of 450 and 390 tokens, hd 64: 102 -> 23.5 us (four steps a wave:
+// the chain from its record to its merge; matrix pipe 21 %). The row layout's loads are ordinary ones: a row's
+// lines are touched by several lanes' loads, and as streaming loads they were fetched again for each (8,000
+// keys at hd 80: 200 -> 140 us).
 //
 // An instance of the row layout or of f32 pages takes every width up to its own: lanes past a row's end
 // hold zeros (K) or re-read the row's first dims into blocks that are never stored (V).
@@ -907,7 +909,8 @@ __device__ __forceinline__ void unit_wave(const PageGeom& g, const UnitGeom& u, 
 }
 
 // Waves per SIMD the register allocator must allow: one where Q, O and a step's operands need more than
-// half the file, four (two workgroups per CU) where they fit a quarter.
+// half the file, four (two workgroups per CU) where they fit a quarter. (Two instances spill, 8 registers
+// to scratch memory each: f16 tiles of hd 256 and f16 rows of 96 dims, both with two column blocks.)
 template <int F, int HDP, int HDVP, int NB>
 constexpr int unit_wpe() {
   using C = Cfg<F, HDP, HDVP, NB>;

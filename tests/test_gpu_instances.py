@@ -7,8 +7,8 @@ identical seeded inputs (the tolerance of test_gpu_parity: max over rows and hea
   Metal sibling's attn_vec instances, misc.metal:82-558; CPU attend / attend_split,
   crates/engine/model/src/forward.rs:585-807);
 - the f32 decode kernel at each width (64, 128, 256) and head group (1, 2, 4, 8, 16), both as split
-  items merged by the merge launch (rows past 16 tiles) and as a row's items merged inside one
-  8-wave workgroup (rows of 3 .. 16 tiles);
+  items merged by the merge launch (rows past 16 tiles; groups of 8 and 16 with explicit split settings)
+  and as a row's items merged inside one 8-wave workgroup (rows of 3 .. 16 tiles);
 - the prefill and mixed launches with P rounded to f16 (prefill_p_f16, the precision of Metal's
   attn_prefill, attn_prefill.metal:17-203) on f16 and bf16 pages at hd 64 and 128, for a Q exact in
   the page type and for a Q with f32 bits (prefill_q_split = 2: one pass of hi + lo products)."""
@@ -57,6 +57,20 @@ def test_decode_f32_every_width_and_group(cuda, hd, group, form):
     w = small("df", "f32", Layer(2 * group, 2, hd, hd), prior=prior, new=[1] * len(prior), seed=67)
     hc, oc, q = pair(w)
     check(w, hc, oc, q, f"f32 hd {hd} group {group} {form}")
+
+
+@pytest.mark.parametrize("hd", [64, 128, 256])
+@pytest.mark.parametrize("group", [8, 16])
+def test_decode_f32_wide_groups_with_split_settings(cuda, hd, group):
+    # long rows of these groups are units by default; explicit split settings keep the f32 decode kernel
+    # and its merge launch
+    w = small("dw", "f32", Layer(2 * group, 2, hd, hd), prior=[600, 40, 250], new=[1] * 3, seed=69)
+    hc, oc, q = pair(w)
+    hc.set_tuning(decode_min_tiles=2)
+    hc.set_timing(True)
+    check(w, hc, oc, q, f"f32 hd {hd} group {group}, split settings")
+    kt = hc.kernel_times()
+    assert kt["decode"][1] == 1 and kt["merge"][1] == 1 and kt["prefill"][1] == 0, kt
 
 
 PF16 = [(kv, hd, mixed, q_kind) for kv in ("f16", "bf16") for hd in (64, 128) for mixed in (False, True)

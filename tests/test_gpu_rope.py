@@ -73,8 +73,8 @@ def test_qk_rope_store_matches_oracle(cuda, case):
     check_case(case, 100 + CASES.index(case), [32760, 0, 1000], [(0, 1), (1, 37), (2, 5)], 40000)
 
 
-# Calls of 1,024 rows or more with no aligned runs of 4 f16 / bf16 rows (q8_0 and f32 pages) take
-# the row kernel of the register path (each row's heads in one workgroup), at each of its widths.
+# Calls of 1,024 rows or more on q8_0 and f32 pages at each width, in aligned runs (those that take the
+# row kernel of the register path: test_gpu_rope_runs.py).
 LONG = [
     ("q8_0", 8, 2, 64, 64, 64, True, True, True, False, 0, False, 1e4),
     ("f32", 8, 2, 128, 128, 128, False, True, False, True, 0, True, 1e6),

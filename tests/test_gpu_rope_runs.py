@@ -29,6 +29,22 @@ def test_runs_match_the_oracle(cuda, case):
     check_case(case, 300 + CASES.index(case), [0, 1, 1000, 14], [(0, 38), (1, 9), (2, 4), (3, 1)], 2048)
 
 
+# 256-wide heads on f32 pages take runs whole from 128 rows on; partly rotated Neox pairs sit in different
+# lanes of the slot kernel, so calls of 1,024 rows or more on q8_0 and f32 pages take the row kernel of the
+# register path (each row's heads in one workgroup), at each of its widths
+LONG = [
+    (("f32", 3, 1, 256, 256, 256, True, True, True, True, 0, False, 1e4), 150),
+    (("q8_0", 8, 2, 64, 64, 32, True, True, True, False, 0, False, 1e4), 1030),
+    (("f32", 8, 2, 128, 128, 64, True, False, True, True, 0, True, 1e6), 1030),
+    (("q8_0", 4, 2, 256, 256, 128, True, True, False, True, 0, False, 1e6), 1030),
+]
+
+
+@pytest.mark.parametrize("case,n", LONG, ids=lambda c: f"{c[0]}-hd{c[3]}-rot{c[5]}" if isinstance(c, tuple) else str(c))
+def test_long_calls_match_the_oracle(cuda, case, n):
+    check_case(case, 400 + n, [0, 500, 0], [(0, n), (1, 3), (2, 1)], 2048)
+
+
 @pytest.mark.parametrize("kv,hd,bt", [("q8_0", 64, 16), ("q8_0", 128, 32), ("q8_0", 256, 16), ("f32", 128, 64)])
 def test_runs_store_the_bytes_single_rows_store(cuda, kv, hd, bt):
     import torch
