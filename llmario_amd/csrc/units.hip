@@ -28,8 +28,8 @@
 // (57 before non-finite V of a masked key was kept out: the masked steps wait for V to test it), bound by the
 // chain of one wave per SIMD's steps and a second, partly filled round of workgroups (waves resident 62 % of
 // the time, issuing VALU 25 % and in the matrix pipe 12 %), two of 2,048: 410 TFLOP/s; hd 80, 32 heads of
-// their own K/V, 8 decode rows and a 120-token chunk: 1,038 -> 30 us (23.5 + merge 4.1; 85 MB; decode rows
-// alone at 8,000 keys: 5.0 TB/s); f32 prompts of 450 and 390 tokens, hd 64: 102 -> 23.5 us (four steps a wave:
+// their own K/V, 8 decode rows and a 120-token chunk: 1,038 -> 29 us (23.5 + merge 4.1; 85 MB; decode rows
+// alone at 8,000 keys: 5.0 TB/s); f32 prompts of 450 and 390 tokens, hd 64: 102 -> 23 us (four steps a wave:
 // the chain from its record to its merge; matrix pipe 21 %). The row layout's loads are ordinary ones: a row's
 // lines are touched by several lanes' loads, and as streaming loads they were fetched again for each (8,000
 // keys at hd 80: 200 -> 140 us).
