@@ -334,7 +334,7 @@ int32_t lmh_bench_read_ceiling(int32_t device, uint64_t bytes, uint32_t iters, d
 /* Test hook (no counterpart in the reference; for CPU tests of the planner, which run under the
  * sanitizers): lmh_attend's work-list planner on host data alone, no device touched. `d` gives a
  * layer geometry as lmh_kv_create takes it, the device facts the planner uses (n_cu; the decode
- * items the device holds at once, 0 = 8 per CU) and a block table [n_seqs][bps] (-1: no block);
+ * items the device holds at once, 0 = 8 per CU; a unit launch: 8 waves per CU) and a block table [n_seqs][bps] (-1: no block);
  * the segments are validated as lmh_attend validates them (every block a row's key range
  * starts or ends in must be in the table). The plan lmh_attend would run is copied out as its
  * internal records: decode items, split-K merges and prefill units (pf_wg lists of pf_per_wg
